@@ -30,7 +30,7 @@ int launch_dense_fp8(const uint8_t* wp, const void* w_s, int w_kind, const uint8
 int launch_dense_fp4(const uint8_t* wp, const uint32_t* wp_s, const uint8_t* xq, const float* xs, bool a_pow2,
                      uint16_t* y, int64_t M, int64_t N, int64_t K, hipStream_t stream);
 bool tile_gemm_fits(int64_t M, int64_t N, int64_t K);
-int launch_tile_gemm(const uint8_t* xq, const float* xs, bool a_pow2, const uint8_t* wp, const void* w_s, int w_kind,
+int launch_tile_gemm(const uint8_t* xq, const void* xs, int a_kind, const uint8_t* wp, const void* w_s, int w_kind,
                      const uint16_t* res, uint16_t* y, uint16_t* y_hi, int64_t n_split, int64_t M, int64_t N,
                      int64_t K, hipStream_t stream);
 
@@ -838,7 +838,7 @@ static int linear_packed(const char* name, const void* x_bf16, const void* w_pac
   if (gemv_mt_serves(M, N, K))
     return gemv_mt_dispatch(xq, xs, qkind, wp, w_s, w_scale_kind, res, y, nullptr, N, M, N, K, pow2, stream);
   if (tile_gemm_fits(M, N, K))
-    return launch_tile_gemm(xq, xs, pow2, wp, w_s, w_scale_kind, res, y, nullptr, N, M, N, K, stream);
+    return launch_tile_gemm(xq, xs, qkind, wp, w_s, w_scale_kind, res, y, nullptr, N, M, N, K, stream);
   return add_residual(res, y, M, N, launch_dense_fp8(wp, w_s, w_scale_kind, xq, xs, pow2, y, M, N, K, stream),
                       stream);
 }
@@ -1234,14 +1234,18 @@ static int gemm_packed(const char* name, const void* a_e4m3, const void* a_s, co
     if (!ws || ws_bytes < need)
       return set_error(WZ_ESPACE, "%s: workspace of %zu bytes needed for M=%lld K=%lld, got %zu", name, need,
                        (long long)M, (long long)K, ws_bytes);
+  }
+  const uint8_t* xq = static_cast<const uint8_t*>(a_e4m3);
+  // the tile GEMM reads e8m0 scales as they are
+  if (tile)
+    return launch_tile_gemm(xq, a_s, act_scale_kind, w, w_s, w_scale_kind, res, c, y_hi, n_split, M, N, K, stream);
+  if (act_scale_kind == WZ_SCALE_UE8M0) {
     const int64_t n = M * (K / 128);
     WZ_LAUNCH("e8m0_to_f32", stream, e8m0_to_f32_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0,
               static_cast<const uint8_t*>(a_s), static_cast<float*>(ws), n);
     if (int rc = check_launch("fp8_gemm_packed scales")) return rc;
     xs = static_cast<const float*>(ws);
   }
-  const uint8_t* xq = static_cast<const uint8_t*>(a_e4m3);
-  if (tile) return launch_tile_gemm(xq, xs, pow2, w, w_s, w_scale_kind, res, c, y_hi, n_split, M, N, K, stream);
   return add_residual(res, c, M, N, launch_dense_fp8(w, w_s, w_scale_kind, xq, xs, pow2, c, M, N, K, stream),
                       stream);
 }
