@@ -231,8 +231,10 @@ int wz_moe_pack_shared(const wz_moe_desc* d, const void* sh_w1, const void* sh_w
 
 /* Bytes of scratch that serve every wz_moe_forward / wz_moe_route call of 1..T
  * tokens (the decode tables of T <= 16 can outgrow a small prefill's needs).
- * T is capped at the chunk that wz_moe_forward runs at once (16384 / k tokens),
- * so the workspace of a long prompt stays that of one chunk. */
+ * T is capped at the chunk that wz_moe_forward runs at once (16384 / k tokens, up
+ * to 65536 / k in a layer of more than 64 experts), so the workspace of a long
+ * prompt stays that of one chunk.  wz_moe_forward also takes a workspace of
+ * 16384 / k tokens' size for any T and then runs chunks of that many. */
 size_t wz_moe_workspace_bytes(const wz_moe_desc* d, int64_t T);
 
 /* Zero the parts of a fresh workspace that must start at zero (arrival
@@ -241,8 +243,8 @@ int wz_moe_workspace_init(void* ws, size_t ws_bytes, hipStream_t stream);
 
 /* Full layer: x_bf16 [T, D], input_ids int64 [T] (read only by hash layers) -> y_bf16 [T, D].
  * Optional routing outputs (may be NULL): weights fp32 [T,k], indices int64 [T,k].
- * Any T: the tokens run in successive chunks of 16384 / k on one workspace
- * (MoE.forward takes any number of tokens, architecture.py:777-794).  A hash id
+ * Any T: the tokens run in successive chunks on one workspace
+ * (wz_moe_workspace_bytes; MoE.forward takes any number of tokens, architecture.py:777-794).  A hash id
  * outside [0, vocab), or a tid2eid entry outside [0, E), gives that token NaN
  * routing weights and a NaN output row (the reference's tid2eid[input_ids]
  * raises); reads stay in bounds. */
@@ -267,7 +269,7 @@ int wz_moe_forward_norm(const wz_moe_desc* d, const void* h_bf16, const float* n
  * serving loops, harnesses that forbid hipMalloc).  The scratch is a device array
  * inside the library, WZ_MOE_NOALLOC_SCRATCH_BYTES (16 MiB) per GPU, held until the
  * process ends: enough for a V4-shape layer (D 4096, I 2048, 256 experts, top-6) up
- * to T = 156 tokens, and for any T where wz_moe_workspace_bytes(d, T) fits.  A larger
+ * to T = 156 tokens, and for any T whose chunk of 16384 / k tokens fits.  A larger
  * call fails with WZ_ESPACE and launches nothing.  The function allocates nothing;
  * its arrival counters are cleared by a fill kernel at the start of every call.
  * All calls on one GPU share its scratch array: calls that overlap on one GPU

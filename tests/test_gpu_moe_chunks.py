@@ -1,0 +1,48 @@
+"""wz_moe_forward's chunks of a long prompt: a layer of many experts takes up to 65536 routed
+pairs at once, a caller whose workspace holds 16384 pairs gets chunks of those.  The layer is
+token-local and every chunk here runs the prefill kernels, so outputs and routing are equal."""
+
+import ctypes
+import dataclasses
+
+import pytest
+import torch
+
+from tests.golden.cases import CASES, make_inputs
+from tests.helpers import bf16_tensor
+from wanferenz_amd import _native as N
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(moe, x, ws):
+    T, dev = x.size(0), moe.device
+    y = torch.empty_like(x)
+    w = torch.empty(T, moe.cfg.topk, device=dev, dtype=torch.float32)
+    i = torch.empty(T, moe.cfg.topk, device=dev, dtype=torch.int64)
+    N.call("wz_moe_workspace_init", ws.data_ptr(), ws.numel(), N.stream_handle(dev))
+    N.call("wz_moe_forward", ctypes.byref(moe.desc), x.data_ptr(), None, T, y.data_ptr(), w.data_ptr(), i.data_ptr(),
+           ws.data_ptr(), ws.numel(), N.stream_handle(dev))
+    return y, w, i
+
+
+# 65536 / 6 = 10922 tokens a chunk at 256 experts (64 count workgroups in the permutation), 5461 at
+# 128; one token more than one full chunk would run the decode kernels, so the rest is >= 17
+@pytest.mark.parametrize("E,T", [(256, 10922), (256, 10942), (128, 5480), (128, 2731 + 16)])
+def test_large_chunks_equal_small_ones(gpu, E, T):
+    from tests.test_gpu_moe import upload_case
+
+    case = dataclasses.replace(CASES["top6_t8"], name=f"chunks_e{E}_t{T}", dim=256, inter=128, n_experts=E, T=T)
+    inp = make_inputs(case)
+    moe = upload_case(case, inp, gpu)
+    x = bf16_tensor(inp.x, gpu)
+    small = 16384 // case.topk
+    need = moe.workspace_bytes(T)
+    assert need > moe.workspace_bytes(small)
+    big = _run(moe, x, torch.empty(need, dtype=torch.uint8, device=gpu))
+    few = _run(moe, x, torch.empty(moe.workspace_bytes(small), dtype=torch.uint8, device=gpu))
+    for a, b in zip(big, few):
+        assert torch.equal(a, b)
+    # sampled rows against calls of their own, 32 tokens each
+    for t in (0, small - 16, T - 32):
+        assert torch.equal(big[0][t:t + 32], moe.forward(x[t:t + 32].contiguous()))

@@ -25,6 +25,7 @@
 //   combine    y[t] = bf16(sum_{experts asc} out[t,e] + shared[t]).
 #include "moe_common.h"
 
+#include <algorithm>
 #include <mutex>
 
 namespace wz {
@@ -278,7 +279,7 @@ __global__ __launch_bounds__(kRouteThreads) void perm_count_kernel(
     int32_t* __restrict__ act_off, int32_t* __restrict__ act_cnt, int32_t* __restrict__ n_active,
     int32_t* __restrict__ mt_u, int32_t* __restrict__ mt_row0, int32_t* __restrict__ mt_n,
     int32_t* __restrict__ n_mt, int mt_cap) {
-  constexpr int kMaxBlocks = kMaxPairs / kRouteThreads;
+  constexpr int kBatch = 16;
   __shared__ int hist[kMaxExperts];
   __shared__ int wsum[128];
   __shared__ int s_last;
@@ -294,23 +295,33 @@ __global__ __launch_bounds__(kRouteThreads) void perm_count_kernel(
   if (tid == 0) s_last = arrive_last(counter, uint32_t(nb)) ? 1 : 0;
   __syncthreads();
   if (!s_last) return;
-  int v[kMaxBlocks];
-#pragma unroll
-  for (int bb = 0; bb < kMaxBlocks; ++bb)
-    v[bb] = (tid < E && bb < nb) ? load_agent_i(cnt + int64_t(bb) * E + tid) : 0;
+  // sixteen workgroups' counts a round trip (read again for their first slots
+  // where there are more: up to 64)
+  int v[kBatch];
   int c = 0;
+  for (int b0 = 0; b0 < nb; b0 += kBatch) {
 #pragma unroll
-  for (int bb = 0; bb < kMaxBlocks; ++bb) c += v[bb];
+    for (int u = 0; u < kBatch; ++u)
+      v[u] = (tid < E && b0 + u < nb) ? load_agent_i(cnt + int64_t(b0 + u) * E + tid) : 0;
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) c += v[u];
+  }
   const int ex = perm_tables(c, E, offsets, active, act_off, act_cnt, n_active, mt_u, mt_row0, mt_n, n_mt, mt_cap,
                              wsum);
   if (tid < E) {
     int run = ex;
+    for (int b0 = 0; b0 < nb; b0 += kBatch) {
+      if (nb > kBatch) {
 #pragma unroll
-    for (int bb = 0; bb < kMaxBlocks; ++bb)
-      if (bb < nb) {
-        base[int64_t(bb) * E + tid] = run;
-        run += v[bb];
+        for (int u = 0; u < kBatch; ++u) v[u] = b0 + u < nb ? load_agent_i(cnt + int64_t(b0 + u) * E + tid) : 0;
       }
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u)
+        if (b0 + u < nb) {
+          base[int64_t(b0 + u) * E + tid] = run;
+          run += v[u];
+        }
+    }
   }
 }
 
@@ -509,10 +520,31 @@ int launch_prefill_experts(const wz_moe_desc* d, const MoeWs& w, const void* x, 
 int launch_prefill_gate(const wz_moe_desc* d, const MoeWs& w, const void* x, const int64_t* input_ids, int64_t T,
                         hipStream_t stream);
 
-// Tokens per call of the kernel sequence: the routed pairs of one call (T * k)
-// fit the kMaxPairs-row tables.  wz_moe_forward serves larger T as successive
-// chunks of this many tokens on the same workspace (the layer is token-local).
-static int64_t chunk_tokens(const wz_moe_desc* d) { return kMaxPairs / d->topk; }
+// Tokens per call of the kernel sequence.  wz_moe_forward serves larger T as successive chunks
+// of this many tokens on the same workspace (the layer is token-local).  Every chunk streams the
+// experts it hits from HBM, so a layer of many experts takes chunks of up to 256 routed rows an
+// expert, where the matrix work of a chunk outweighs its weights: 6000 tokens over 256 MXFP4
+// experts of 2048 are one chunk instead of three and read 3.4 GB instead of 10 (2794 -> 1867 us
+// a layer).  A layer of few experts keeps kMaxPairs, and so does a call whose workspace holds no
+// more (its size before).  The bounds keep a chunk's operands addressable by 32-bit buffer
+// offsets and its tokens by one grid dimension.
+static int64_t small_chunk_tokens(const wz_moe_desc* d) { return kMaxPairs / d->topk; }
+
+static int64_t chunk_tokens(const wz_moe_desc* d) {
+  const int64_t k = d->topk, pairs = std::min<int64_t>(int64_t(256) * d->n_experts, kMaxChunkPairs);
+  int64_t t = std::min<int64_t>(pairs / k, 32768);
+  t = std::min(t, ((int64_t(1) << 31) - 1) / std::max<int64_t>(d->dim, 1));
+  t = std::min(t, ((int64_t(1) << 31) - 1) / ((k + 1) * std::max<int64_t>(d->inter, 1)));
+  return std::max(t, small_chunk_tokens(d));
+}
+
+// Workspace of every call of 1 .. T tokens in chunks of up to `chunk` tokens.
+static size_t ws_bytes_of(const wz_moe_desc* d, int64_t T, int64_t chunk) {
+  T = std::min(T, chunk);
+  const size_t big = moe_ws_layout(d, T, nullptr).bytes;
+  const size_t dec = moe_ws_layout(d, T < kDecodeMaxT ? T : kDecodeMaxT, nullptr).bytes;
+  return big > dec ? big : dec;
+}
 
 static int validate(const wz_moe_desc* d, int64_t T, const void* ws, size_t ws_bytes,
                     const char* what, bool chunked = false) {
@@ -538,7 +570,7 @@ static int validate(const wz_moe_desc* d, int64_t T, const void* ws, size_t ws_b
   }
   if (T == 0) return WZ_OK;  // nothing to do: no workspace needed
   if (!ws) return set_error(WZ_EINVAL, "%s: null workspace", what);
-  const size_t need = wz_moe_workspace_bytes(d, T);
+  const size_t need = ws_bytes_of(d, T, small_chunk_tokens(d));
   if (ws_bytes < need)
     return set_error(WZ_ESPACE, "%s: workspace %zu bytes < %zu needed for T=%lld", what, ws_bytes,
                      need, (long long)T);
@@ -572,7 +604,7 @@ static int launch_routing(const wz_moe_desc* d, const MoeWs& w, const void* x,
   // the gate scores are spent once the top-k is chosen: their [T, E] floats hold
   // the per-workgroup counts and first slots ([nb, E] each; P > 1024 makes T >= 64)
   const int nb = int((P + kRouteThreads - 1) / kRouteThreads);
-  if (int64_t(2) * nb * E > T * E || nb > kMaxPairs / kRouteThreads)
+  if (int64_t(2) * nb * E > T * E || nb > kMaxChunkPairs / kRouteThreads)
     return set_error(WZ_EINVAL, "moe perm: %d count blocks do not fit the score buffer (T=%lld)", nb, (long long)T);
   int32_t* cnt = reinterpret_cast<int32_t*>(w.scores);
   int32_t* base = cnt + int64_t(nb) * E;
@@ -589,10 +621,7 @@ static int launch_routing(const wz_moe_desc* d, const MoeWs& w, const void* x,
 
 extern "C" size_t wz_moe_workspace_bytes(const wz_moe_desc* d, int64_t T) {
   if (!d || T < 0 || d->topk <= 0) return 0;
-  if (T > wz::chunk_tokens(d)) T = wz::chunk_tokens(d);
-  const size_t big = wz::moe_ws_layout(d, T, nullptr).bytes;
-  const size_t dec = wz::moe_ws_layout(d, T < wz::kDecodeMaxT ? T : wz::kDecodeMaxT, nullptr).bytes;
-  return big > dec ? big : dec;
+  return wz::ws_bytes_of(d, T, wz::chunk_tokens(d));
 }
 
 __global__ void zero_words_kernel(uint32_t* p, int n) {
@@ -671,7 +700,9 @@ extern "C" int wz_moe_forward(const wz_moe_desc* d, const void* x_bf16, const in
   if (!d->sh_w1_s || !d->sh_w3_s || !d->sh_w2_s)
     return set_error(WZ_EINVAL, "moe_forward: shared-expert block scales missing");
   if (d->tid2eid && !input_ids) return set_error(WZ_EINVAL, "moe: hash-routed layer needs input_ids");
-  const int64_t C = chunk_tokens(d), k = d->topk, D = d->dim;
+  const int64_t k = d->topk, D = d->dim;
+  int64_t C = chunk_tokens(d);
+  if (ws_bytes < ws_bytes_of(d, T, C)) C = small_chunk_tokens(d);
   for (int64_t t0 = 0; t0 < T; t0 += C) {
     const int64_t n = T - t0 < C ? T - t0 : C;
     if (int rc = forward_chunk(d, static_cast<const uint16_t*>(x_bf16) + t0 * D, input_ids ? input_ids + t0 : nullptr,
@@ -773,7 +804,7 @@ extern "C" int wz_moe_forward_noalloc(const wz_moe_desc* d, const void* x_bf16, 
   if (d->topk <= 0 || d->topk > 16) return set_error(WZ_EINVAL, "moe_forward_noalloc: topk=%d outside 1..16", d->topk);
   if (T < 0) return set_error(WZ_EINVAL, "moe_forward_noalloc: T=%lld < 0", (long long)T);
   if (T == 0) return WZ_OK;
-  const size_t need = wz_moe_workspace_bytes(d, T);
+  const size_t need = ws_bytes_of(d, T, small_chunk_tokens(d));
   if (need > size_t(WZ_MOE_NOALLOC_SCRATCH_BYTES))
     return set_error(WZ_ESPACE,
                      "moe_forward_noalloc: this layer at T=%lld needs %zu bytes of scratch, more than the %d "

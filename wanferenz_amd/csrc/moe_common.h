@@ -7,7 +7,8 @@ namespace wz {
 
 constexpr int kRouteThreads = 1024;
 constexpr int kMaxExperts = 512;
-constexpr int kMaxPairs = 16384;
+constexpr int kMaxPairs = 16384;      // routed pairs of a call of the kernel sequence (wz_moe_route, stage replays)
+constexpr int kMaxChunkPairs = 65536;  // ... of wz_moe_forward's chunks for layers of many experts (chunk_tokens)
 constexpr int kGateTok = 8;
 constexpr int kDecodeMaxT = 16;       // tokens served by the decode kernels
 constexpr int kNormMaxT = 8;          // rows the decode route launch normalises itself (fused ffn norm)
