@@ -4,9 +4,8 @@ oracle's restatement of torch_ops.py:114-146.
 Bar: bf16 outputs within max|d|/max|ref| <= 1e-2 and cosine >= 0.9999 (the kernels
 multiply a bf16 P by V, as the reference's GPU kernel does, reference.py:404-405;
 the CPU reference keeps P in fp32); queries the reference turns into NaN (no valid
-index in the first block of 64) are NaN here.  Head counts that are a multiple of
-64 run the 64-head kernel, split over workgroups with a workspace when there are
-few queries; others the 16-head kernel.
+index in the first block of 64) are NaN here.  A workgroup holds one, two or four
+tiles of 16 heads, and few queries are split over workgroups with a workspace.
 """
 
 import numpy as np
@@ -122,3 +121,19 @@ def test_running_max_moves(gpu, h, d, s):
     scale = d ** -0.5
     ref = om.sparse_attn(q, kv, sink, idx, scale)
     _check(_run(gpu, q, kv, sink, idx, scale), ref)
+
+
+@pytest.mark.parametrize("h", [16, 32, 48, 64, 80])
+@pytest.mark.parametrize("s", [1, 260])
+def test_head_groups_and_empty_blocks(gpu, h, s):
+    """Each number of head tiles a workgroup can hold (one, two, four with the last one
+    missing, a second group of one), split over workgroups and not, with blocks that have no
+    valid index first-but-one, in the middle and last: they are skipped and add nothing."""
+    d, topk = 512, 64 * 6 + 5
+    q, kv, sink, idx = _inputs(31 + h + s, 1, s, h, d, 300, topk, invalid=0.3)
+    idx[..., 0] = np.maximum(idx[..., 0], 0)
+    idx[:, ::2, 64:128] = -1
+    idx[:, 1::3, 192:320] = -1
+    idx[:, ::4, 384:] = -1
+    scale = d ** -0.5
+    _check(_run(gpu, q, kv, sink, idx, scale), om.sparse_attn(q, kv, sink, idx, scale))

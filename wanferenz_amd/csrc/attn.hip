@@ -30,17 +30,24 @@ __device__ __forceinline__ v4f mfma_bf16_32(v8s_t a, v8s_t b, v4f c) {
 __host__ __device__ constexpr int64_t attn_part_floats(int d) { return 128 + 64 * int64_t(d); }
 
 // LDS image of one block of 64 KV rows, row-major, no padding.  The 16-byte
-// chunks of row r sit XOR-swizzled (chunk c at slot c ^ swz(r)), so that both
-// read patterns are free of bank conflicts: 16 rows reading one chunk (the K
-// operand of S^T) land on 16 distinct 4-bank groups, and 8 rows reading two
-// adjacent chunks (the transpose reads of V) on 16 distinct groups as well.
+// chunks of row r sit XOR-swizzled (chunk c at slot c ^ swz(r)) so that both
+// read patterns are free of bank conflicts.  A 16-byte read of one chunk of
+// 16 rows (the K operand of S^T) is served in passes of 16 lanes that mix rows
+// 0-3 and 12-15 of one lane group with rows 4-11 of the next, whose chunk is
+// the neighbour: the slots of rows 0-3 and 12-15 are closed under ^ 1, so the
+// passes' slots are distinct (without that, every pass took two turns: 45 % of
+// the LDS cycles).  The transpose reads of V take two adjacent chunks of 8
+// consecutive rows, which have distinct slot pairs.
 template <int D>
 struct KsLayout {
   static constexpr int RB = 2 * D;             // bytes per row
   static constexpr int RPI = 1024 / RB;        // rows per 1 KB load
   static constexpr int NG = kAttnBlock / RPI;  // loads per block
   static constexpr int BYTES = kAttnBlock * RB;
-  static __device__ __forceinline__ int swz(int row) { return ((row & 7) << 1) ^ ((row >> 3) & 1); }
+  static __device__ __forceinline__ int swz(int row) {
+    const int hi = (row >> 3) & 1;
+    return ((row ^ (hi << 2)) & 7) << 1 | hi;
+  }
   // byte address of element `col` (a multiple of 4) of `row`
   static __device__ __forceinline__ int at(int row, int col) {
     return row * RB + (((col >> 3) ^ swz(row)) << 4) + ((col & 7) << 1);
@@ -59,46 +66,58 @@ __device__ __forceinline__ uint32_t cvt_bf16x2(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{a, b}, bf16x2_t));
 }
 
-// One workgroup per (query, 64 heads, range of 64-index blocks), 4 waves;
-// wave w owns heads 64 hq + 16w .. +16 (a wave whose head group is past H only
-// helps load).  Per block:
-//   * the 64 gathered KV rows sit in LDS row-major ([row][d], padded); they
-//     were loaded while the previous block was computed (double buffer);
-//   * S^T[64 rows, 16 heads] = K Q^T with V_MFMA_F32_16X16X32_BF16, K from
-//     LDS, the wave's Q fragments in registers for the launch.  The transposed
-//     product leaves lane (head n, group g) holding rows 16rt + 4g + i, which
-//     is the A-operand layout of P in P V once two row tiles are paired
-//     (k slots 0-3: rows 32kc + 4g + i, slots 4-7: rows 32kc + 16 + 4g + i):
-//     P never leaves registers and the softmax needs no other wave;
+// One workgroup per (query, up to 64 heads, range of 64-index blocks), 8 waves, HT tiles of
+// 16 heads.  The LDS reads of the KV rows are what bounds a block, so the waves split both
+// products such that a row is read as few times as the registers allow: with Q and O of 64
+// heads held in registers, K twice, V once and P once a wave, 256 KB a block of 64 rows
+// (2048 cycles at 128 B per cycle, as long as its MFMAs); four waves of 16 heads each, which
+// read every row of K and V themselves, took 512 KB and 3.5 us a block, where this takes 2.5.
+// 2048 queries of a prompt from position 0 (64 heads of 512, 6.5 of 10 blocks with valid
+// indices): 346 -> 174 us, of which 57 us are the workgroups' starts and ends (Q in and O out,
+// 268 MB) that one workgroup a CU does not overlap with its products; 640 valid indices for each
+// of 2048 queries 347 -> 264 us.
+//   * the 64 gathered KV rows sit in LDS row-major; they were loaded while the previous block
+//     was computed (double buffer).  A block without a valid index (a prompt's early positions
+//     have fewer selected rows than slots) adds nothing and is skipped;
+//   * S^T = K Q^T with V_MFMA_F32_16X16X32_BF16: wave w has rows 16 (w & 3) .. +16 and SHT
+//     head tiles.  Lane (head n, group g) then holds rows 16rt + 4g + i, four consecutive k
+//     slots of the P operand below (k slots 0-3: rows 32kc + 4g + i, slots 4-7: rows 32kc +
+//     16 + 4g + i), and P goes to LDS in that operand's order, 8 bytes a lane;
 //   * P = exp(S - m) in bf16 (the GPU reference also multiplies a bf16 P,
-//     reference.py:404-405), with m moved only when a block's maximum exceeds
-//     it by more than kLazyMax (P <= e^8; the final division by the sum taken
-//     with the same m makes the result independent of m);
-//   * O[16 heads, D] += P V, the V operand read from the row-major rows with
-//     the LDS transpose read (ds_read_b64_tr_b16: in each 16-lane group, lane
-//     i addressing row base + (i >> 2), column c0 + 4(i & 3) makes lane j
-//     receive rows base..base+3 of column c0 + j).
-// A workgroup that covers every block normalises (sink term included) and
-// stores bf16; for few queries the blocks are split over workgroups that
-// store (m, l, O) partials and sparse_attn_combine_kernel merges them.
-template <int D, bool SPLIT>
-__global__ __launch_bounds__(256, 1) void sparse_attn_kernel(const uint16_t* __restrict__ q,
-                                                            const uint16_t* __restrict__ kv,
-                                                            const float* __restrict__ sink,
-                                                            const int32_t* __restrict__ idx,
-                                                            uint16_t* __restrict__ o, float* __restrict__ part, int S,
-                                                            int H, int N, int topk, int bps, int nsplit,
-                                                            float scale) {
-  using L = KsLayout<D>;
-  constexpr int KC = D / 32;  // 32-wide d chunks of S
-  constexpr int NT = D / 16;  // 16-column tiles of O
-  static_assert(L::NG % 4 == 0, "a block's loads must split evenly over the 4 waves");
-  static_assert(L::RB / 16 >= 16, "the swizzle permutes 16 chunks of a row");
-  __shared__ __align__(16) uint8_t ksb[2][L::BYTES];
-  __shared__ int s_idx[kAttnIdxCap];
-  __shared__ int s_any;
+//     reference.py:404-405), with m moved only when a block's maximum exceeds it by more than
+//     kLazyMax (P <= e^8; the final division by the sum taken with the same m makes the result
+//     independent of m).  Every wave writes its P with the m of the blocks before and flags a
+//     head that needs a new one; only then a second barrier follows, after the maxima have
+//     met, O is rescaled and P written again;
+//   * O^T[D, heads] += V^T P^T: wave w has columns w D/8 .. +D/8 of every head, V read from
+//     the row-major rows with the LDS transpose read (ds_read_b64_tr_b16: in each 16-lane
+//     group, lane i addressing row base + (i >> 2), column c0 + 4(i & 3) makes lane j receive
+//     rows base..base+3 of column c0 + j).  A lane holds four consecutive columns of one head.
+// A workgroup that covers every block normalises (sink term included) and stores bf16, whole
+// lines through LDS; for few queries the blocks are split over workgroups that store (m, l, O)
+// partials and sparse_attn_combine_kernel merges them.
+constexpr int kAttnWaves = 8;
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+template <int D, int HT, bool SPLIT>
+__global__ __launch_bounds__(64 * kAttnWaves, 2) void sparse_attn_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ kv, const float* __restrict__ sink,
+    const int32_t* __restrict__ idx, uint16_t* __restrict__ o, float* __restrict__ part, int S, int H, int N, int topk,
+    int bps, int nsplit, float scale) {
+  using L = KsLayout<D>;
+  constexpr int KC = D / 32;                  // 32-wide d chunks of S
+  constexpr int NT = D / 16 / kAttnWaves;     // 16-column tiles of O per wave
+  constexpr int SHT = HT == 4 ? 2 : 1;        // head tiles of S per wave
+  constexpr int NL = L::NG / kAttnWaves;      // loads of a block per wave
+  constexpr int kNoRow = int(0x80000000u / L::RB);  // an unused index: its byte offset lies past any cache
+  static_assert(L::NG % kAttnWaves == 0, "a block's loads must split evenly over the waves");
+  static_assert(L::RB / 16 >= 16, "the swizzle permutes 16 chunks of a row");
+  __shared__ __align__(1024) uint8_t ksb[2][L::BYTES];
+  __shared__ __align__(16) uint8_t s_p[2][16 * HT][64];  // [kc][head]: group g's 8 k slots at 16 g
+  __shared__ int s_idx[kAttnIdxCap];
+  __shared__ float s_max[4][64], s_l[4][64];  // [row tile][head]
+  __shared__ int s_bump[kAttnIdxCap / kAttnBlock], s_used[kAttnIdxCap / kAttnBlock];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nl = lane & 15, g = lane >> 4;
   const int HQ = (H + 63) / 64;
   const int c = blockIdx.x % nsplit, qh = blockIdx.x / nsplit;
@@ -106,185 +125,263 @@ __global__ __launch_bounds__(256, 1) void sparse_attn_kernel(const uint16_t* __r
   const int nblk = (topk + kAttnBlock - 1) / kAttnBlock;
   const int blk0 = c * bps, blk1 = min(blk0 + bps, nblk);
   const int nb = blk1 - blk0;  // >= 1: the host never launches an empty split
-  const int hg0 = hq * 64 + 16 * wave;
-  const bool active = hg0 < H;  // H % 16 == 0: the whole head group exists
+  const int h0 = hq * 64;
+  const int rt = wave & 3, ht0 = (wave >> 2) * SHT;  // this wave's row tile and first head tile of S
+  const bool has_s = ht0 < HT;
 
-  // Q fragments first (they do not wait for the indices; B operand of S^T): lane (head nl, group g) holds d 32cc + 8g .. +8
-  v8s_t qb[KC];
-  const uint16_t* qrow = q + (int64_t(bs) * H + (active ? hg0 : 0) + nl) * D;
-#pragma unroll
-  for (int cc = 0; cc < KC; ++cc) qb[cc] = *reinterpret_cast<const v8s_t*>(qrow + 32 * cc + 8 * g);
-
-  const int32_t* ib = idx + int64_t(bs) * topk + int64_t(blk0) * kAttnBlock;
-  if (tid == 0) s_any = 0;
-  for (int j = tid; j < nb * kAttnBlock; j += 256) {
-    const int v = blk0 * kAttnBlock + j < topk ? ib[j] : -1;
-    s_idx[j] = (v >= 0 && v < N) ? v : -1;
+  // Q rows into the second buffer, in the layout of a block: read from memory once in whole
+  // lines, where fragments loaded by the four waves that share them took 4 us more a
+  // workgroup; heads past H repeat the last one and are dropped
+  const uint32_t ks_lds = lds_addr(&ksb[0][0]);
+  const __amdgpu_buffer_rsrc_t q_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(q + int64_t(bs) * H * D), short(0), H * L::RB, 0x00020000);
+  for (int gi = wave; gi < 16 * HT / L::RPI; gi += kAttnWaves) {
+    const int row = gi * L::RPI + lane / (L::RB / 16), slot = lane % (L::RB / 16);
+    load_lds_16(q_rsrc, __builtin_amdgcn_readfirstlane(ks_lds + L::BYTES + gi * 1024),
+                uint32_t(min(h0 + row, H - 1)) * L::RB + ((slot ^ L::swz(row)) << 4));
   }
-  __syncthreads();
-  if (blk0 == 0 && tid < kAttnBlock && s_idx[tid] >= 0) s_any = 1;
+  const int32_t* ib = idx + int64_t(bs) * topk + int64_t(blk0) * kAttnBlock;
+  for (int j = tid; j < nb * kAttnBlock; j += 64 * kAttnWaves) {
+    const int v = blk0 * kAttnBlock + j < topk ? ib[j] : -1;
+    const bool ok = v >= 0 && v < N;
+    s_idx[j] = ok ? v : kNoRow;
+    const uint64_t m = __ballot(ok);  // a wave covers one whole block
+    if (lane == 0) {
+      s_used[j >> 6] = m != 0;
+      s_bump[j >> 6] = 0;
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // Q and the indices are in LDS
+  uint32_t todo = uint32_t(__ballot(lane < nb && s_used[min(lane, nb - 1)] != 0));  // nb <= 32
+  const bool poisoned = blk0 == 0 && !(todo & 1u);
 
-  // rows of block t -> ksb[t & 1]; an unused index reads past the end of the
+  // rows of block t -> ksb[buf]; an unused index reads past the end of the
   // buffer, which returns zeros (the reference zero-fills those rows)
   const __amdgpu_buffer_rsrc_t kv_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint16_t*>(kv + int64_t(b) * N * D), short(0), int(int64_t(N) * L::RB), 0x00020000);
-  const uint32_t ks_lds = uint32_t(uintptr_t((__attribute__((address_space(3))) uint8_t*)&ksb[0][0]));
   // Load gi of a block fills rows gi * RPI .. +RPI; lane i writes slot i & (RB/16 - 1)
   // of row gi * RPI + i / (RB/16), so it fetches that row's chunk slot ^ swz(row).
-  auto issue = [&](int t) {
-    const int rin = lane / (L::RB / 16), slot = lane % (L::RB / 16);
-    int ri[L::NG / 4];  // every row index first: the asm loads below order memory accesses
+  auto issue = [&](int t, int buf) {
+    int ln = lane;
+    asm volatile("" : "+v"(ln));  // recomputed for each block: the registers go to Q and O
+    const int rin = ln / (L::RB / 16), slot = ln % (L::RB / 16);
+    int ri[NL];  // every row index first: the asm loads below order memory accesses
 #pragma unroll
-    for (int j = 0; j < L::NG / 4; ++j) ri[j] = s_idx[t * kAttnBlock + (j * 4 + wave) * L::RPI + rin];
+    for (int j = 0; j < NL; ++j) ri[j] = s_idx[t * kAttnBlock + (j * kAttnWaves + wave) * L::RPI + rin];
 #pragma unroll
-    for (int j = 0; j < L::NG / 4; ++j) {
-      const int gi = j * 4 + wave, row = gi * L::RPI + rin;
-      const uint32_t vo = ri[j] < 0 ? 0x80000000u : uint32_t(ri[j]) * L::RB + ((slot ^ L::swz(row)) << 4);
-      load_lds_16(kv_rsrc, __builtin_amdgcn_readfirstlane(ks_lds + (t & 1) * L::BYTES + gi * 1024), vo);
+    for (int j = 0; j < NL; ++j) {
+      const int gi = j * kAttnWaves + wave, row = gi * L::RPI + rin;
+      const uint32_t vo = uint32_t(ri[j]) * L::RB + ((slot ^ L::swz(row)) << 4);
+      load_lds_16(kv_rsrc, __builtin_amdgcn_readfirstlane(ks_lds + buf * L::BYTES + gi * 1024), vo);
     }
   };
-  issue(0);
-
-  v4f acc[NT];  // acc[nt][i] = O[head 4g + i][16nt + nl]
+  if (todo) issue(__builtin_ctz(todo), 0);
+  // Q fragments (B operand of S^T): lane (head nl, group g) holds d 32cc + 8g .. +8
+  v8s_t qb[SHT][KC];
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt) acc[nt] = v4f{0.f, 0.f, 0.f, 0.f};
-  float m_use = -INFINITY, l_run = 0.0f;  // head nl: running max, this lane's share of the sum
+  for (int h = 0; h < SHT; ++h)
+#pragma unroll
+    for (int cc = 0; cc < KC; ++cc)
+      qb[h][cc] = *reinterpret_cast<const v8s_t*>(ksb[1] + L::at(16 * (has_s ? ht0 + h : 0) + nl, 32 * cc + 8 * g));
 
-  for (int t = 0; t < nb; ++t) {
+  v4f acc[HT][NT];  // acc[ht][nt][i] = O[head 16ht + nl][w D/8 + 16nt + 4g + i]
+#pragma unroll
+  for (int ht = 0; ht < HT; ++ht)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) acc[ht][nt] = v4f{0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY;  // running max of head `lane`, the same in every wave
+  float m_s[SHT], l_s[SHT];  // of this lane's heads of S: the max, and its rows' share of the sum
+#pragma unroll
+  for (int h = 0; h < SHT; ++h) {
+    m_s[h] = -INFINITY;
+    l_s[h] = 0.0f;
+  }
+
+  int buf = 0;
+#pragma unroll 1
+  for (bool first = true; todo; first = false, buf ^= 1) {
+    const int t = __builtin_ctz(todo);
+    todo &= todo - 1;
     __builtin_amdgcn_s_waitcnt(0);  // this wave's loads of block t have landed
-    __syncthreads();                // ... and every wave's; block t - 1's buffer is free
-    if (t + 1 < nb) issue(t + 1);
-    const uint8_t* ks = ksb[t & 1];
-    const uint64_t vmask = __ballot(s_idx[t * kAttnBlock + lane] >= 0);
-    if (!active) continue;
+    __syncthreads();                // ... and every wave's; the other buffer and s_p are free
+    if (todo) issue(__builtin_ctz(todo), buf ^ 1);
+    const uint8_t* const ks = ksb[buf];
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
+    const int nl = ln & 15, g = ln >> 4;
 
-    // ---- S^T[rows, 16 heads]: sacc[rt][i] = S[row 16rt + 4g + i][head nl] ----
-    // K fragments are read two d chunks ahead of their MFMAs (three buffers)
-    v4f sacc[4];
+    // ---- S^T[16 rows, heads]: sacc[h][i] = S[row 16rt + 4g + i][head nl of tile h] ----
+    v4f sacc[SHT];
+    float p_sum[SHT];
+    // P = exp(S - m) in bf16 to LDS, this lane's part of the row sum to p_sum
+    auto put_p = [&]() {
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) sacc[rt] = v4f{0.f, 0.f, 0.f, 0.f};
-    v8s_t kf[3][4];
-    auto kload = [&](int cc, v8s_t* dst) {
+      for (int h = 0; h < SHT; ++h) {
+        float pv[4];
 #pragma unroll
-      for (int rt = 0; rt < 4; ++rt)
-        dst[rt] = *reinterpret_cast<const v8s_t*>(ks + L::at(16 * rt + nl, 32 * cc + 8 * g));
-    };
-    kload(0, kf[0]);
-    kload(1, kf[1]);
-#pragma unroll
-    for (int cc = 0; cc < KC; ++cc) {
-      if (cc + 2 < KC) kload(cc + 2, kf[(cc + 2) % 3]);
-      __builtin_amdgcn_sched_barrier(0);  // keep the reads two chunks ahead of their use
-#pragma unroll
-      for (int rt = 0; rt < 4; ++rt) sacc[rt] = mfma_bf16_32(kf[cc % 3][rt], qb[cc], sacc[rt]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    float bmax = -INFINITY;
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int row = 16 * rt + 4 * g + i;
-        sacc[rt][i] = (vmask >> row) & 1 ? sacc[rt][i] * scale : -INFINITY;
-        bmax = fmaxf(bmax, sacc[rt][i]);
+        for (int i = 0; i < 4; ++i) pv[i] = sacc[h][i] == -INFINITY ? 0.0f : __expf(sacc[h][i] - m_s[h]);
+        p_sum[h] = (pv[0] + pv[1]) + (pv[2] + pv[3]);
+        *reinterpret_cast<uint2*>(&s_p[rt >> 1][16 * (ht0 + h) + nl][16 * g + 8 * (rt & 1)]) =
+            make_uint2(cvt_bf16x2(pv[0], pv[1]), cvt_bf16x2(pv[2], pv[3]));
       }
-    bmax = fmaxf(bmax, __shfl_xor(bmax, 16, kWave));
-    bmax = fmaxf(bmax, __shfl_xor(bmax, 32, kWave));
-    const bool bump = bmax > m_use + kLazyMax;
-    if (__ballot(bump)) {
-      const float m_new = bump ? bmax : m_use;
-      const bool fresh = m_use == -INFINITY;  // nothing accumulated yet for this head
-      const float resc = !bump ? 1.0f : (fresh ? 0.0f : __expf(m_use - m_new));
-      l_run *= resc;
-      m_use = m_new;
-      // O[h, :] *= resc(h) on the matrix core, so the accumulators stay where the
-      // P V products keep them: O += A_i B_i (V_MFMA_F32_16X16X4_F32, k = lane
-      // group g) with B_i[g][n] = O[4g + i][n] (component i of each lane) and
-      // A_i[m][g] = resc(m) - 1 where m = 4g + i, else 0; step i only changes
-      // rows = i (mod 4), which later steps do not read.  Skipped while every
-      // bumped head is fresh (its accumulators are still zero).
-      if (__ballot(bump && !fresh)) {
+    };
+    if (has_s) {
+      const uint64_t vmask = __ballot(s_idx[t * kAttnBlock + lane] != kNoRow);
+#pragma unroll
+      for (int h = 0; h < SHT; ++h) sacc[h] = v4f{0.f, 0.f, 0.f, 0.f};
+      // K fragments are read kAhead d chunks ahead of their MFMAs
+      constexpr int kAhead = 3;
+      // chunk (4cc + g) ^ swz: its low four bits, and 16 chunks (256 bytes) a step of the rest
+      const int krow = (16 * rt + nl) * L::RB, kchunk = (g ^ L::swz(nl)) << 4;
+      v8s_t kf[kAhead + 1];
+      auto kload = [&](int cc) {
+        kf[cc % (kAhead + 1)] = *reinterpret_cast<const v8s_t*>(ks + krow + ((4 * (cc & 3)) << 4 ^ kchunk) + (cc >> 2) * 256);
+      };
+#pragma unroll
+      for (int cc = 0; cc < kAhead; ++cc) kload(cc);
+#pragma unroll
+      for (int cc = 0; cc < KC; ++cc) {
+        if (cc + kAhead < KC) kload(cc + kAhead);
+        __builtin_amdgcn_sched_barrier(0);  // keep the reads ahead of their use
+#pragma unroll
+        for (int h = 0; h < SHT; ++h) sacc[h] = mfma_bf16_32(kf[cc % (kAhead + 1)], qb[h][cc], sacc[h]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      bool bump = false;
+#pragma unroll
+      for (int h = 0; h < SHT; ++h) {
+        float bmax = -INFINITY;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const float ai = nl == 4 * g + i ? resc - 1.0f : 0.0f;
+          sacc[h][i] = (vmask >> (16 * rt + 4 * g + i)) & 1 ? sacc[h][i] * scale : -INFINITY;
+          bmax = fmaxf(bmax, sacc[h][i]);
+        }
+        bmax = fmaxf(bmax, __shfl_xor(bmax, 16, kWave));
+        bmax = fmaxf(bmax, __shfl_xor(bmax, 32, kWave));
+        bump |= bmax > m_s[h] + kLazyMax;
+        if (g == 0) s_max[rt][16 * (ht0 + h) + nl] = bmax;
+      }
+      if (__ballot(bump)) {
+        if (lane == 0) s_bump[t] = 1;
+      }
+      if (!first) put_p();
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the loads of the next block stay in flight
+    if (first || s_bump[t]) {
+      // the block's maxima have met: head `lane`
+      const int hl = lane < 16 * HT ? lane : 0;
+      const float bm = fmaxf(fmaxf(s_max[0][hl], s_max[1][hl]), fmaxf(s_max[2][hl], s_max[3][hl]));
+      const bool bump = bm > m_run + kLazyMax;
+      // nothing accumulated yet for a head without a maximum
+      const float resc = !bump ? 1.0f : (m_run == -INFINITY ? 0.0f : __expf(m_run - bm));
+      m_run = bump ? bm : m_run;
 #pragma unroll
-          for (int nt = 0; nt < NT; ++nt)
-            acc[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(ai, acc[nt][i], acc[nt], 0, 0, 0);
+      for (int h = 0; h < SHT; ++h) {
+        m_s[h] = __shfl(m_run, (16 * (ht0 + h) + nl) & 63, kWave);
+        l_s[h] *= __shfl(resc, (16 * (ht0 + h) + nl) & 63, kWave);
+      }
+      if (!first) {
+#pragma unroll
+        for (int ht = 0; ht < HT; ++ht) {
+          const float r = __shfl(resc, 16 * ht + nl, kWave);
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt) acc[ht][nt] = acc[ht][nt] * r;
         }
       }
+      if (has_s) put_p();
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     }
-    v8s_t pa[2];
+    if (has_s) {
 #pragma unroll
-    for (int kc = 0; kc < 2; ++kc) {
-      float pv[8];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        pv[i] = sacc[2 * kc][i] == -INFINITY ? 0.0f : __expf(sacc[2 * kc][i] - m_use);
-        pv[4 + i] = sacc[2 * kc + 1][i] == -INFINITY ? 0.0f : __expf(sacc[2 * kc + 1][i] - m_use);
-        l_run += pv[i] + pv[4 + i];
-      }
-      const uint4 u = make_uint4(cvt_bf16x2(pv[0], pv[1]), cvt_bf16x2(pv[2], pv[3]), cvt_bf16x2(pv[4], pv[5]),
-                                 cvt_bf16x2(pv[6], pv[7]));
-      pa[kc] = __builtin_bit_cast(v8s_t, u);
+      for (int h = 0; h < SHT; ++h) l_s[h] += p_sum[h];
     }
 
-    // ---- O[16 heads, D] += P[16 heads, 64 rows] V[64 rows, D] ----
-    // V fragments are read two column tiles ahead of their MFMAs (three buffers)
-    v8s_t vf[3][2];
-    auto vload = [&](int nt, v8s_t* dst) {
-      const int col = 16 * nt + 4 * (nl & 3);
-#pragma unroll
-      for (int kc = 0; kc < 2; ++kc) {
-        const int row = 32 * kc + 4 * g + (nl >> 2);
-        const v4s_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t*)(ks + L::at(row, col)));
-        const v4s_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t*)(ks + L::at(row + 16, col)));
-        dst[kc] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-      }
+    // ---- O^T[wave's columns, heads] += V^T[columns, 64 rows] P^T[64 rows, heads] ----
+    // V fragments are read two column tiles ahead of their MFMAs
+    v8s_t vf[3];
+    const int vrow = 4 * g + (nl >> 2);  // rows 16 apart share their swizzle
+    auto vload = [&](int j) {  // j = kc NT + nt
+      const uint8_t* const p = ks + L::at(vrow, wave * 16 * NT + 16 * (j % NT) + 4 * (nl & 3)) + (j / NT) * 32 * L::RB;
+      const v4s_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t*)p);
+      const v4s_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t*)(p + 16 * L::RB));
+      vf[j % 3] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
     };
-    vload(0, vf[0]);
-    vload(1, vf[1]);
+    v8s_t pb[HT];  // of 32 rows kc; the second half's are read as the first half's are used up
+    auto pload = [&](int kc, int ht) {
+      pb[ht] = *reinterpret_cast<const v8s_t*>(&s_p[kc][16 * ht + nl][16 * g]);
+    };
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      if (nt + 2 < NT) vload(nt + 2, vf[(nt + 2) % 3]);
+    for (int ht = 0; ht < HT; ++ht) pload(0, ht);
+    vload(0);
+    vload(1);
+#pragma unroll
+    for (int j = 0; j < 2 * NT; ++j) {
+      if (j + 2 < 2 * NT) vload(j + 2);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int kc = 0; kc < 2; ++kc) acc[nt] = mfma_bf16_32(pa[kc], vf[nt % 3][kc], acc[nt]);
+      for (int ht = 0; ht < HT; ++ht) {
+        acc[ht][j % NT] = mfma_bf16_32(vf[j % 3], pb[ht], acc[ht][j % NT]);
+        if (j == NT - 1) {
+          __builtin_amdgcn_sched_barrier(0);
+          pload(1, ht);
+        }
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
   }
-  if (!active) return;
 
-  l_run += __shfl_xor(l_run, 16, kWave);
-  l_run += __shfl_xor(l_run, 32, kWave);
-  const bool poisoned = blk0 == 0 && s_any == 0;
-  if (!SPLIT) {
-    // normalise by the sum (sink term included): one reciprocal per head, then
-    // products (within 1 fp32 ulp of the quotient, before the bf16 rounding)
+  if (has_s) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int hd = hg0 + 4 * g + i;
-      const float lh = __shfl(l_run, 4 * g + i, kWave), mh = __shfl(m_use, 4 * g + i, kWave);
-      const float inv = poisoned ? __builtin_nanf("") : 1.0f / (lh + __expf(sink[hd] - mh));
-      uint16_t* orow = o + (int64_t(bs) * H + hd) * D;
+    for (int h = 0; h < SHT; ++h) {
+      l_s[h] += __shfl_xor(l_s[h], 16, kWave);
+      l_s[h] += __shfl_xor(l_s[h], 32, kWave);
+      if (g == 0) s_l[rt][16 * (ht0 + h) + nl] = l_s[h];
+    }
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  const int hl = lane < 16 * HT ? lane : 0;
+  const float l_run = (s_l[0][hl] + s_l[1][hl]) + (s_l[2][hl] + s_l[3][hl]);  // of head `lane`
+  if constexpr (!SPLIT) {
+    // normalise by the sum (sink term included): one reciprocal per head, then products
+    // (within 1 fp32 ulp of the quotient, before the bf16 rounding); the tile goes out through
+    // this wave's part of the buffer that the last block did not use, 16-byte chunks
+    // XOR-swizzled by row
+    const float inv_l =
+        poisoned ? __builtin_nanf("") : 1.0f / (l_run + __expf(sink[min(h0 + hl, H - 1)] - m_run));
+    constexpr int RB = 32 * NT, NCH = RB / 16;  // bytes and chunks of the wave's columns of a head
+    uint8_t* const so = ksb[buf] + wave * (16 * HT * RB);
 #pragma unroll
-      for (int nt = 0; nt < NT; nt += 2) {
-        const uint32_t pr = cvt_bf16x2(acc[nt][i] * inv, acc[nt + 1][i] * inv);
-        orow[16 * nt + nl] = uint16_t(pr & 0xFFFFu);
-        orow[16 * nt + 16 + nl] = uint16_t(pr >> 16);
+    for (int ht = 0; ht < HT; ++ht) {
+      const float inv = __shfl(inv_l, 16 * ht + nl, kWave);
+      const int row = 16 * ht + nl;
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) {
+        const int ch = 2 * nt + (g >> 1);
+        const v4f v = acc[ht][nt] * inv;
+        *reinterpret_cast<uint2*>(so + row * RB + ((ch ^ (row & (NCH - 1))) << 4) + (g & 1) * 8) =
+            make_uint2(cvt_bf16x2(v[0], v[1]), cvt_bf16x2(v[2], v[3]));
       }
     }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    uint16_t* const ow = o + (int64_t(bs) * H + h0) * D + wave * 16 * NT;
+#pragma unroll
+    for (int it = 0; it < (16 * HT * NCH + 63) / 64; ++it) {
+      const int row = it * (64 / NCH) + lane / NCH, ch = lane % NCH;
+      if (row >= 16 * HT || h0 + row >= H) continue;
+      *reinterpret_cast<v4i*>(ow + int64_t(row) * D + ch * 8) =
+          *reinterpret_cast<const v4i*>(so + row * RB + ((ch ^ (row & (NCH - 1))) << 4));
+    }
   } else {
-    float* pp = part + int64_t(blockIdx.x) * attn_part_floats(D);
-    if (g == 0) {
-      pp[16 * wave + nl] = m_use;
-      pp[64 + 16 * wave + nl] = poisoned ? __builtin_nanf("") : l_run;
+    float* const pp = part + int64_t(blockIdx.x) * attn_part_floats(D);
+    if (wave == 0) {
+      pp[lane] = m_run;
+      pp[64 + lane] = poisoned ? __builtin_nanf("") : l_run;
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      float* orow = pp + 128 + int64_t(16 * wave + 4 * g + i) * D;
+    for (int ht = 0; ht < HT; ++ht)
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) orow[16 * nt + nl] = acc[nt][i];
-    }
+      for (int nt = 0; nt < NT; ++nt)
+        *reinterpret_cast<v4f*>(pp + 128 + int64_t(16 * ht + nl) * D + (wave * NT + nt) * 16 + 4 * g) = acc[ht][nt];
   }
 }
 
@@ -366,21 +463,31 @@ static inline AttnSplit attn_split(int64_t units, int64_t topk) {
   return {nsplit, bps};
 }
 
-template <int D>
+template <int D, int HT>
 static int launch_attn(const uint16_t* q, const uint16_t* kv, const float* sink, const int32_t* idx, uint16_t* o,
                        float* part, int64_t units, int S, int H, int N, int topk, AttnSplit sp, float scale,
                        hipStream_t stream) {
   if (sp.nsplit == 1) {
-    WZ_LAUNCH("sparse_attn", stream, (sparse_attn_kernel<D, false>), dim3{unsigned(units)}, dim3(256), 0, q, kv,
+    WZ_LAUNCH("sparse_attn", stream, (sparse_attn_kernel<D, HT, false>), dim3{unsigned(units)}, dim3(64 * kAttnWaves), 0, q, kv,
               sink, idx, o, part, S, H, N, topk, sp.bps, 1, scale);
     return check_launch("sparse_attn");
   }
-  WZ_LAUNCH("sparse_attn", stream, (sparse_attn_kernel<D, true>), dim3{unsigned(units * sp.nsplit)}, dim3(256), 0, q,
+  WZ_LAUNCH("sparse_attn", stream, (sparse_attn_kernel<D, HT, true>), dim3{unsigned(units * sp.nsplit)}, dim3(64 * kAttnWaves), 0, q,
             kv, sink, idx, o, part, S, H, N, topk, sp.bps, sp.nsplit, scale);
   if (int rc = check_launch("sparse_attn")) return rc;
   WZ_LAUNCH("sparse_attn_combine", stream, sparse_attn_combine_kernel<D>, dim3{unsigned(units * 16)}, dim3(256), 0,
             part, sink, o, H, sp.nsplit);
   return check_launch("sparse_attn_combine");
+}
+
+// Head tiles of a workgroup: the heads of a group of 64 that exist.
+template <int D>
+static int launch_attn_heads(const uint16_t* q, const uint16_t* kv, const float* sink, const int32_t* idx, uint16_t* o,
+                             float* part, int64_t units, int S, int H, int N, int topk, AttnSplit sp, float scale,
+                             hipStream_t stream) {
+  if (H <= 16) return launch_attn<D, 1>(q, kv, sink, idx, o, part, units, S, H, N, topk, sp, scale, stream);
+  if (H <= 32) return launch_attn<D, 2>(q, kv, sink, idx, o, part, units, S, H, N, topk, sp, scale, stream);
+  return launch_attn<D, 4>(q, kv, sink, idx, o, part, units, S, H, N, topk, sp, scale, stream);
 }
 
 }  // namespace wz
@@ -434,11 +541,11 @@ extern "C" int wz_sparse_attn(const void* q_bf16, const void* kv_bf16, const flo
   uint16_t* o = static_cast<uint16_t*>(o_bf16);
   float* part = static_cast<float*>(workspace);
   if (D == 512)
-    return launch_attn<512>(q, kv, attn_sink, topk_idxs, o, part, units, int(S), int(H), int(N), int(topk), sp,
-                            softmax_scale, stream);
+    return launch_attn_heads<512>(q, kv, attn_sink, topk_idxs, o, part, units, int(S), int(H), int(N), int(topk), sp,
+                                  softmax_scale, stream);
   if (D == 256)
-    return launch_attn<256>(q, kv, attn_sink, topk_idxs, o, part, units, int(S), int(H), int(N), int(topk), sp,
-                            softmax_scale, stream);
-  return launch_attn<128>(q, kv, attn_sink, topk_idxs, o, part, units, int(S), int(H), int(N), int(topk), sp,
-                          softmax_scale, stream);
+    return launch_attn_heads<256>(q, kv, attn_sink, topk_idxs, o, part, units, int(S), int(H), int(N), int(topk), sp,
+                                  softmax_scale, stream);
+  return launch_attn_heads<128>(q, kv, attn_sink, topk_idxs, o, part, units, int(S), int(H), int(N), int(topk), sp,
+                                softmax_scale, stream);
 }
