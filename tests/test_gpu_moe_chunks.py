@@ -46,3 +46,24 @@ def test_large_chunks_equal_small_ones(gpu, E, T):
     # sampled rows against calls of their own, 32 tokens each
     for t in (0, small - 16, T - 32):
         assert torch.equal(big[0][t:t + 32], moe.forward(x[t:t + 32].contiguous()))
+
+
+# the wide routed tiles (1024 tokens and 32 pair rows an expert on) against calls below them, whose
+# rows are in 64-row tiles: a partial last N-block of w2 (640 columns), five K-blocks (a ragged
+# group of scales), experts of many tiles and of few rows, a skewed selection with empty experts
+@pytest.mark.parametrize("E,T,skew", [(5, 1024, 0.0), (40, 1111, 0.0), (64, 1500, 0.05), (17, 2100, 1.0)])
+def test_wide_tiles_equal_narrow_ones(gpu, E, T, skew):
+    from tests.test_gpu_moe import upload_case
+
+    case = dataclasses.replace(CASES["top6_t8"], name=f"wide_e{E}_t{T}", dim=640, inter=384, n_experts=E, topk=2, T=T)
+    inp = make_inputs(case)
+    moe = upload_case(case, inp, gpu)
+    if skew:
+        moe.weights.gate_bias.copy_(torch.linspace(skew, -skew, E))
+    x = bf16_tensor(inp.x, gpu)
+    y, w, i = _run(moe, x, torch.empty(moe.workspace_bytes(T), dtype=torch.uint8, device=gpu))
+    for at in range(0, T, 700):
+        n = min(700, T - at)
+        ws = torch.empty(moe.workspace_bytes(n), dtype=torch.uint8, device=gpu)
+        for a, b in zip((y, w, i), _run(moe, x[at:at + n].contiguous(), ws)):
+            assert torch.equal(a[at:at + n], b)

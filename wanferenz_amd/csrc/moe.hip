@@ -208,13 +208,13 @@ __device__ __forceinline__ int block_excl_scan(int v, int* wsum, int& total) {
 // The permutation's tables from each expert's pair count c (thread e of the
 // block holds expert e; E <= 1024 = block size): offsets and the active-expert
 // list (offsets, counts), and the M-tile table of the prefill GEMMs (each
-// active expert's pair rows cut into tiles of kPrefillTileRows, in active
+// active expert's pair rows cut into tiles of mt_rows, in active
 // order).  Returns the expert's first slot.
 __device__ int perm_tables(int c, int E, int32_t* __restrict__ offsets, int32_t* __restrict__ active,
                            int32_t* __restrict__ act_off, int32_t* __restrict__ act_cnt,
                            int32_t* __restrict__ n_active, int32_t* __restrict__ mt_u,
                            int32_t* __restrict__ mt_row0, int32_t* __restrict__ mt_n, int32_t* __restrict__ n_mt,
-                           int mt_cap, int* wsum) {
+                           int mt_rows, int mt_cap, int* wsum) {
   const int tid = threadIdx.x;
   int total;
   const int ex = block_excl_scan(c, wsum, total);
@@ -233,13 +233,13 @@ __device__ int perm_tables(int c, int E, int32_t* __restrict__ offsets, int32_t*
     offsets[E] = total;
     n_active[0] = nact;
   }
-  const int ntile = flag ? (c + kPrefillTileRows - 1) / kPrefillTileRows : 0;
+  const int ntile = flag ? (c + mt_rows - 1) / mt_rows : 0;
   int ntiles;
   const int mt0 = block_excl_scan(ntile, wsum, ntiles);
   for (int i = 0; i < ntile && mt0 + i < mt_cap; ++i) {
     mt_u[mt0 + i] = u;
-    mt_row0[mt0 + i] = ex + i * kPrefillTileRows;
-    mt_n[mt0 + i] = min(kPrefillTileRows, c - i * kPrefillTileRows);
+    mt_row0[mt0 + i] = ex + i * mt_rows;
+    mt_n[mt0 + i] = min(mt_rows, c - i * mt_rows);
   }
   if (tid == 0) n_mt[0] = min(ntiles, mt_cap);
   return ex;
@@ -278,7 +278,7 @@ __global__ __launch_bounds__(kRouteThreads) void perm_count_kernel(
     uint32_t* __restrict__ counter, int32_t* __restrict__ offsets, int32_t* __restrict__ active,
     int32_t* __restrict__ act_off, int32_t* __restrict__ act_cnt, int32_t* __restrict__ n_active,
     int32_t* __restrict__ mt_u, int32_t* __restrict__ mt_row0, int32_t* __restrict__ mt_n,
-    int32_t* __restrict__ n_mt, int mt_cap) {
+    int32_t* __restrict__ n_mt, int mt_rows, int mt_cap) {
   constexpr int kBatch = 16;
   __shared__ int hist[kMaxExperts];
   __shared__ int wsum[128];
@@ -306,8 +306,8 @@ __global__ __launch_bounds__(kRouteThreads) void perm_count_kernel(
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) c += v[u];
   }
-  const int ex = perm_tables(c, E, offsets, active, act_off, act_cnt, n_active, mt_u, mt_row0, mt_n, n_mt, mt_cap,
-                             wsum);
+  const int ex = perm_tables(c, E, offsets, active, act_off, act_cnt, n_active, mt_u, mt_row0, mt_n, n_mt, mt_rows,
+                             mt_cap, wsum);
   if (tid < E) {
     int run = ex;
     for (int b0 = 0; b0 < nb; b0 += kBatch) {
@@ -373,7 +373,7 @@ __global__ __launch_bounds__(kRouteThreads) void perm_kernel(const int32_t* __re
                                                              int32_t* __restrict__ pos, int32_t* __restrict__ mt_u,
                                                              int32_t* __restrict__ mt_row0,
                                                              int32_t* __restrict__ mt_n, int32_t* __restrict__ n_mt,
-                                                             int mt_cap) {
+                                                             int mt_rows, int mt_cap) {
   constexpr int kW = kRouteThreads / 64;  // waves
   __shared__ int wcnt[kW][kMaxExperts];   // pairs of expert e in wave w's chunk, then their first slot
   __shared__ int wsum[128];
@@ -392,8 +392,8 @@ __global__ __launch_bounds__(kRouteThreads) void perm_kernel(const int32_t* __re
   int c = 0;
   if (tid < E)
     for (int w = 0; w < kW; ++w) c += wcnt[w][tid];
-  const int ex = perm_tables(c, E, offsets, active, act_off, act_cnt, n_active, mt_u, mt_row0, mt_n, n_mt, mt_cap,
-                             wsum);
+  const int ex = perm_tables(c, E, offsets, active, act_off, act_cnt, n_active, mt_u, mt_row0, mt_n, n_mt, mt_rows,
+                             mt_cap, wsum);
   if (tid < E) {
     int run = ex;
     for (int w = 0; w < kW; ++w) {
@@ -515,6 +515,7 @@ __global__ void export_routing_kernel(const MoeWs ws, int P, float* __restrict__
 
 int launch_decode(const wz_moe_desc* d, const MoeWs& w, const void* x, const int64_t* ids, int64_t T,
                   void* y, hipStream_t stream, int only, const float* nw = nullptr, float eps = 0.0f);
+int prefill_tile_rows(const wz_moe_desc* d, int64_t T);
 int launch_prefill_experts(const wz_moe_desc* d, const MoeWs& w, const void* x, int64_t T, hipStream_t stream,
                            int only);
 int launch_prefill_gate(const wz_moe_desc* d, const MoeWs& w, const void* x, const int64_t* input_ids, int64_t T,
@@ -595,10 +596,11 @@ static int launch_routing(const wz_moe_desc* d, const MoeWs& w, const void* x,
     if (int rc = check_launch("moe topk")) return rc;
   }
   const int64_t P = T * k, mt_cap = P / kPrefillTileRows + (P < E ? P : E) + 1;
+  const int mt_rows = prefill_tile_rows(d, T);
   if (P <= kRouteThreads) {
     WZ_LAUNCH("moe_perm", stream, perm_kernel, dim3(1), dim3(kRouteThreads), 0, w.idx, int(T), E, k, w.offsets,
               w.active, w.act_off, w.act_cnt, w.n_active, w.perm_token, w.perm_slot, w.pos, w.mt_u, w.mt_row0,
-              w.mt_n, w.n_mt, int(mt_cap));
+              w.mt_n, w.n_mt, mt_rows, int(mt_cap));
     return check_launch("moe perm");
   }
   // the gate scores are spent once the top-k is chosen: their [T, E] floats hold
@@ -610,7 +612,7 @@ static int launch_routing(const wz_moe_desc* d, const MoeWs& w, const void* x,
   int32_t* base = cnt + int64_t(nb) * E;
   WZ_LAUNCH("moe_perm", stream, perm_count_kernel, dim3(unsigned(nb)), dim3(kRouteThreads), 0, w.idx, int(T), E, k,
             cnt, base, &w.counters[kCounterWords - 1], w.offsets, w.active, w.act_off, w.act_cnt, w.n_active,
-            w.mt_u, w.mt_row0, w.mt_n, w.n_mt, int(mt_cap));
+            w.mt_u, w.mt_row0, w.mt_n, w.n_mt, mt_rows, int(mt_cap));
   if (int rc = check_launch("moe perm count")) return rc;
   WZ_LAUNCH("moe_perm", stream, perm_place_kernel, dim3(unsigned(nb)), dim3(kRouteThreads), 0, w.idx, int(T), E, k,
             base, w.perm_token, w.perm_slot, w.pos);

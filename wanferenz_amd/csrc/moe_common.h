@@ -14,6 +14,7 @@ constexpr int kDecodeMaxT = 16;       // tokens served by the decode kernels
 constexpr int kNormMaxT = 8;          // rows the decode route launch normalises itself (fused ffn norm)
 constexpr int kNormMaxD = 4096;       // and their width
 constexpr int kPrefillTileRows = 64;  // pair rows per M-tile of the prefill / dense GEMMs
+constexpr int kPrefillWideRows = 128;  // ... of the wide routed tiles (prefill_tile_rows)
 constexpr int kCounterWords = 4096;   // arrival counters at the start of the workspace
 
 // Scratch of one MoE layer call, carved from the caller's workspace.  The

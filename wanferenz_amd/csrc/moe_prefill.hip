@@ -2,7 +2,7 @@
 // canonical (expert, token, slot) pair order produced by the routing kernels.
 //
 //   (the routing's perm_kernel also cuts each active expert's pair rows into
-//   M-tiles of 64 rows)
+//   M-tiles of 64 rows; of 128 where the wide tiles below run)
 //   xquant    act_quant(x) once for all experts (quant.hip).
 //   w13       per (M-tile, 64 intermediate features): the gathered 128 fp8
 //             activation rows of one 128-wide K-block are staged in LDS; each
@@ -20,6 +20,10 @@
 // Semantics: Expert.forward / MoE.forward of wanferenz/model/architecture.py
 // (w1/w3 outputs rounded to bf16, clamp, silu(g)*u*weight -> bf16 -> w2).
 #include "moe_common.h"
+
+#include <algorithm>
+#include <atomic>
+#include <type_traits>
 
 namespace wz {
 
@@ -1018,6 +1022,285 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(2))) 
   }
 }
 
+// ------------------------------------------------------------ wide tiles ---
+//
+// Routed w1/w3 (+ SwiGLU + act_quant of h) and w2 over M-tiles of up to 128 pair rows, with
+// power-of-two activation scales (the accumulators chain over K, the bits of gemm_tile_body).
+// The 64-row tiles above are bound by what the CUs draw from L2: a K-step brings 8 KB of rows
+// and 16 KB of weights for 64 x 256 outputs (w2: 8 + 8 KB for 64 x 128), 10.8 GB a launch at
+// 6000 tokens, at about 10 TB/s.  Here eight waves share both operands through LDS, 16 KB of
+// rows and 16 KB of weights for 128 x 256 outputs: two thirds of the bytes for w1/w3, half
+// for w2.  Waves are 2 along M x 4 along N; the tile's 16-row groups are dealt evenly over
+// the two, so a tile of any height keeps both busy.  A wave's four weight tiles are the
+// MFMA's first operand: a lane then holds four consecutive columns of one row, and codes and
+// bf16 rows go out through LDS in whole lines.  Two workgroups a CU, one K-block in flight
+// each: the loads of K-block q + 1 go out after the barrier that frees its buffer, ahead of
+// the products of q.  Three K-blocks in flight at one workgroup a CU took 1122 us where this
+// takes 831: more waves hide more than more loads.  What bounds it now: half of the wave
+// cycles wait for loads (the experts' weights come from beyond L2), the matrix cores are busy
+// 40 %.  M-tiles in order, each with all its N-blocks (788 us for w1/w3 against 838 in groups
+// of 8 x 8).  6000 tokens over 256 experts, w1/w3 and w2 with the shared expert: 1061 + 574 ->
+// 955 + 451 us, the layer 1840 -> 1553; 2048 tokens with skewed experts 920 -> 863.
+constexpr int kWideThreads = 512;
+constexpr int kWideStage = kPrefillWideRows * 128 + 16 * 1024;  // rows, then 16 weight tiles
+constexpr int kWideScales = 16 * 256;                           // weight scales of 4 K-blocks
+
+static inline size_t wide_lds(int K) { return 2 * kWideStage + 2 * kWideScales + size_t((K / 128 + 3) / 4) * 4 * kPrefillWideRows; }
+
+template <bool W13>
+__global__ __launch_bounds__(kWideThreads, 4) void prefill_wide_kernel(wz_moe_desc d, MoeWs ws, int T, int nblk) {
+  extern __shared__ __align__(1024) uint8_t st[];  // two stages, two groups of weight scales, row scales [KG][128][4]
+  uint8_t* const sc = st + 2 * kWideStage;
+  uint8_t* const as_l = sc + 2 * kWideScales;
+  const int n = ws.n_mt[0] * nblk;
+  if (int(blockIdx.x) >= n) return;
+  const int t = xcd_runs(int(blockIdx.x), 0, n), mt = t / nblk, nt = t % nblk;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nl = lane & 15, g = lane >> 4, wm = wave >> 2, wn = wave & 3;
+  const int D = d.dim, I = d.inter, k = d.topk, P = T * k, E = d.n_experts;
+  const int K = W13 ? D : I, KB = K / 128, KG = (KB + 3) / 4;
+  const int NCT = (W13 ? I : D) / 16;  // 16-column tiles of the output
+  const int e = clampi(ws.active[clampi(ws.mt_u[mt], 0, E - 1)], 0, E - 1);
+  const int row0 = clampi(ws.mt_row0[mt], 0, P);
+  const int nrows = clampi(ws.mt_n[mt], 0, min(kPrefillWideRows, P - row0));
+  if (nrows <= 0) return;
+  const int n16 = (nrows + 15) / 16, nm0 = (n16 + 1) / 2;
+  const int m_first = wm ? nm0 : 0, nm = wm ? n16 - nm0 : nm0;  // this wave's 16-row groups
+
+  // rows past nrows repeat the last one, their outputs are dropped
+  auto src_of = [&](int r) {
+    const int p = row0 + min(r, nrows - 1);
+    return W13 ? clampi(ws.perm_token[p], 0, T - 1) : p;
+  };
+  // the wave's direct loads of a K-block: rows 16w .. 16w + 15 (against an empty range where
+  // none exists) and weight tiles 2w, 2w + 1, with their scales every fourth K-block
+  const int64_t a_rows = W13 ? T : P + T;
+  const __amdgpu_buffer_rsrc_t a_rs = __builtin_amdgcn_make_buffer_rsrc(
+      W13 ? ws.xq : ws.hq, short(0), 16 * wave < nrows ? int(a_rows * K) : 0, 0x00020000);
+  const int64_t tile_bytes = int64_t(NCT) * KB * (W13 ? 2048 : 1024);  // of one expert
+  const int64_t scale_bytes = int64_t(NCT) * KG * (W13 ? 512 : 256);
+  const uint8_t* const wb = static_cast<const uint8_t*>(W13 ? d.w13p : d.w2p) + e * tile_bytes;
+  const uint8_t* const sb0 = reinterpret_cast<const uint8_t*>(W13 ? d.w13p_s : d.w2p_s) + e * scale_bytes;
+  const __amdgpu_buffer_rsrc_t b_rs =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(wb), short(0), int(tile_bytes), 0x00020000);
+  const __amdgpu_buffer_rsrc_t s_rs =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(sb0), short(0), int(scale_bytes), 0x00020000);
+  uint32_t avo[2], bvo[2], svo[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int row = 16 * wave + 8 * j + (lane >> 3);
+    avo[j] = uint32_t(src_of(row)) * uint32_t(K) + uint32_t(((lane & 7) ^ a_swz(row)) << 4);
+    if (W13) {  // feature tile 8 nt + w: w1, then w3
+      bvo[j] = uint32_t(nt * 8 + wave) * uint32_t(KB) * 2048u + uint32_t(j) * 1024u + uint32_t(lane) * 16u;
+      svo[j] = uint32_t(nt * 8 + wave) * uint32_t(KG) * 512u + uint32_t(j) * 256u + uint32_t(lane) * 4u;
+    } else {
+      const int c = min(nt * 16 + 2 * wave + j, NCT - 1);  // tiles past the last column repeat it
+      bvo[j] = uint32_t(c) * uint32_t(KB) * 1024u + uint32_t(lane) * 16u;
+      svo[j] = uint32_t(c) * uint32_t(KG) * 256u + uint32_t(lane) * 4u;
+    }
+  }
+  const uint32_t lds0 = lds_addr(st);
+  auto issue = [&](int q) {
+    const uint32_t sa = lds0 + uint32_t(q & 1) * kWideStage + uint32_t(wave) * 2048u;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      load_lds_16(a_rs, __builtin_amdgcn_readfirstlane(sa + j * 1024), avo[j], uint32_t(q) * 128u);
+      load_lds_16(b_rs, __builtin_amdgcn_readfirstlane(sa + kPrefillWideRows * 128 + j * 1024), bvo[j],
+                  uint32_t(q) * (W13 ? 2048u : 1024u));
+    }
+    if ((q & 3) == 0) {
+      const uint32_t ss = lds0 + 2 * kWideStage + uint32_t((q >> 2) & 1) * kWideScales + uint32_t(wave) * 512u;
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        load_lds_4(s_rs, __builtin_amdgcn_readfirstlane(ss + j * 256), svo[j], uint32_t(q >> 2) * (W13 ? 512u : 256u));
+    }
+  };
+  issue(0);
+
+  // the row scales of the whole K range as e8m0 bytes
+  const uint32_t* const xs = reinterpret_cast<const uint32_t*>(W13 ? ws.xs : ws.hs);
+  for (int i = tid; i < n16 * 16 * KB; i += kWideThreads) {
+    const int r = i / KB, kb = i - r * KB;
+    as_l[((kb >> 2) * kPrefillWideRows + r) * 4 + (kb & 3)] = uint8_t((xs[int64_t(src_of(r)) * KB + kb] >> 23) & 0xFFu);
+  }
+
+  v4f acc[4][4];  // acc[m][c][i] = row 16 (m_first + m) + nl, column 4g + i of weight tile 4 wn + c
+#pragma unroll
+  for (int m = 0; m < 4; ++m)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[m][c] = v4f{0.f, 0.f, 0.f, 0.f};
+  // the K loop of a wave with NM 16-row groups (every wave passes the same barriers)
+  auto k_loop = [&](auto groups) {
+    constexpr int NM = decltype(groups)::value;
+    uint32_t wse[4] = {}, ase[4] = {};  // e8m0 scales of four K-blocks, the current one's in the low byte
+    for (int q = 0; q < KB; ++q) {
+      // K-block q has landed, and every wave has read K-block q - 1: its buffer takes q + 1
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      if (q + 1 < KB) issue(q + 1);
+      if constexpr (NM > 0) {
+        const uint8_t* const sa = st + (q & 1) * kWideStage;
+        const uint8_t* const sb = sa + kPrefillWideRows * 128 + wn * 4096 + lane * 16;
+        if ((q & 3) == 0) {
+          const uint8_t* const ss = sc + ((q >> 2) & 1) * kWideScales + wn * 1024 + lane * 4;
+          const uint8_t* const pas = as_l + ((q >> 2) * kPrefillWideRows + m_first * 16 + nl) * 4;
+#pragma unroll
+          for (int c = 0; c < 4; ++c) wse[c] = *reinterpret_cast<const uint32_t*>(ss + c * 256);
+#pragma unroll
+          for (int m = 0; m < NM; ++m) ase[m] = *reinterpret_cast<const uint32_t*>(pas + m * 64);
+        } else {
+#pragma unroll
+          for (int c = 0; c < 4; ++c) wse[c] >>= 8;
+#pragma unroll
+          for (int m = 0; m < NM; ++m) ase[m] >>= 8;
+        }
+        v8i bv[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const v4i w = *reinterpret_cast<const v4i*>(sb + c * 1024);
+          bv[c] = v8i{w[0], w[1], w[2], w[3], 0, 0, 0, 0};
+        }
+        // a 16-row group's rows are read ahead of the products of the group before
+        const uint8_t* const pa = sa + (m_first * 16 + nl) * 128;  // rows 16 apart share their swizzle
+        const int o = (g ^ a_swz(nl)) << 4;
+        v8i av[2];
+        auto rows = [&](int m) {
+          const v4i lo = *reinterpret_cast<const v4i*>(pa + o + m * 2048);
+          const v4i hi = *reinterpret_cast<const v4i*>(pa + (o ^ 64) + m * 2048);
+          av[m & 1] = v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        };
+        rows(0);
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+          if (m + 1 < NM) rows(m + 1);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int c = 0; c < 4; ++c)
+            acc[m][c] = mfma_scaled<kFmtFp4, kFmtFp8>(bv[c], av[m & 1], acc[m][c], int(wse[c]), int(ase[m]));
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+  };
+  if (nm == 4)
+    k_loop(std::integral_constant<int, 4>());
+  else if (nm == 3)
+    k_loop(std::integral_constant<int, 3>());
+  else if (nm == 2)
+    k_loop(std::integral_constant<int, 2>());
+  else if (nm == 1)
+    k_loop(std::integral_constant<int, 1>());
+  else
+    k_loop(std::integral_constant<int, 0>());
+  __syncthreads();  // the stages are free
+
+  if constexpr (W13) {
+    // h = SwiGLU times the routing weight, rounded to bf16 as the expert's intermediate is
+    // (architecture.py:739-741), then act_quant (torch_ops.py:33-49): the workgroup's 128
+    // features are one quantisation block, whose amax the four waves of a row meet in LDS
+    float* const am_s = reinterpret_cast<float*>(st);
+    uint8_t* const so = st + 4 * kPrefillWideRows * 4;
+    float wts[4], am[4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      const int p = row0 + min((m_first + m) * 16 + nl, nrows - 1);
+      wts[m] = ws.weights[int64_t(clampi(ws.perm_token[p], 0, T - 1)) * k + clampi(ws.perm_slot[p], 0, k - 1)];
+    }
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      if (m >= nm) continue;
+      const int r = (m_first + m) * 16 + nl;
+      am[m] = 0.0f;
+#pragma unroll
+      for (int c = 0; c < 4; c += 2)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float gv = bf16_round(acc[m][c][i]), uv = bf16_round(acc[m][c + 1][i]);
+          if (d.swiglu_limit > 0.0f) {
+            uv = clamp_keep_nan(uv, -d.swiglu_limit, d.swiglu_limit);
+            gv = gv > d.swiglu_limit ? d.swiglu_limit : gv;
+          }
+          const float hv = bf16_round(wts[m] * (silu_f32(gv) * uv));
+          acc[m][c][i] = hv;
+          am[m] = absmax(am[m], hv);
+        }
+      am[m] = wave_absmax_xor(am[m], 16);
+      am[m] = wave_absmax_xor(am[m], 32);
+      if (g == 0) am_s[wn * kPrefillWideRows + r] = am[m];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      if (m >= nm) continue;
+      const int r = (m_first + m) * 16 + nl;
+      float amax = am[m];
+#pragma unroll
+      for (int w = 0; w < 4; ++w) amax = absmax(amax, am_s[w * kPrefillWideRows + r]);
+      const ActScale s = act_scale(amax, true);
+#pragma unroll
+      for (int c = 0; c < 4; c += 2)
+        *reinterpret_cast<uint32_t*>(so + r * 128 + (((2 * wn + (c >> 1)) ^ (r & 7)) << 4) + 4 * g) =
+            pack_fp8x4(quant_div(acc[m][c][0], s, true), quant_div(acc[m][c][1], s, true),
+                       quant_div(acc[m][c][2], s, true), quant_div(acc[m][c][3], s, true));
+      if (wn == 0 && g == 0 && r < nrows) ws.hs[int64_t(row0 + r) * (I / 128) + nt] = s.s;
+    }
+    __syncthreads();
+    for (int i = tid; i < nrows * 8; i += kWideThreads) {
+      const int r = i >> 3, ch = i & 7;
+      *reinterpret_cast<v4i*>(ws.hq + int64_t(row0 + r) * I + nt * 128 + ch * 16) =
+          *reinterpret_cast<const v4i*>(so + r * 128 + ((ch ^ (r & 7)) << 4));
+    }
+  } else {
+    uint8_t* const so = st + wave * 8192;  // the wave's rows x 64 columns in bf16
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      if (m >= nm) continue;
+      const int r = m * 16 + nl;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int ch = 2 * c + (g >> 1);
+        *reinterpret_cast<uint2*>(so + r * 128 + ((ch ^ (r & 7)) << 4) + (g & 1) * 8) =
+            make_uint2(f32x2_to_bf16x2(acc[m][c][0], acc[m][c][1]), f32x2_to_bf16x2(acc[m][c][2], acc[m][c][3]));
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const int col = nt * 256 + wn * 64 + (lane & 7) * 8;
+    for (int r = lane >> 3; r < nm * 16; r += 8) {
+      const int gr = m_first * 16 + r;
+      if (gr < nrows && col < D)
+        *reinterpret_cast<v4i*>(ws.out2 + int64_t(row0 + gr) * D + col) =
+            *reinterpret_cast<const v4i*>(so + r * 128 + (((lane & 7) ^ (r & 7)) << 4));
+    }
+  }
+}
+
+template <bool W13>
+static int launch_wide(const wz_moe_desc* d, const MoeWs& w, int64_t T, int nblk, hipStream_t stream) {
+  const size_t lds = wide_lds(W13 ? d->dim : d->inter);
+  static std::atomic<int> granted{0};
+  if (int(lds) > granted.load(std::memory_order_relaxed)) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_wide_kernel<W13>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)) != hipSuccess)
+      return set_error(WZ_ELAUNCH, "moe prefill: %zu bytes of LDS refused", lds);
+    granted.store(int(lds), std::memory_order_relaxed);
+  }
+  const int64_t P = T * d->topk, E = d->n_experts;
+  const int64_t mt_max = P / kPrefillWideRows + std::min(P, E) + 1;
+  WZ_LAUNCH(W13 ? "moe_w13" : "moe_w2", stream, prefill_wide_kernel<W13>, dim3(unsigned(mt_max * nblk)),
+            dim3(kWideThreads), lds, *d, w, int(T), nblk);
+  return check_launch(W13 ? "moe w13" : "moe w2");
+}
+
+// Pair rows per M-tile of a prefill of T tokens.  Wide tiles from 1024 tokens and 32 rows an
+// expert on, where both sides cross (256 experts of 4096 x 2048, us a layer, 64-row against
+// wide tiles): 16 rows 640 / 683, 24 rows 734 / 734, 35 rows 804 / 785, 48 rows 882 / 850,
+// 141 rows 1868 / 1589.  With fewer rows the launch streams weights from memory, and the
+// 64-row tiles keep three K-blocks in flight.
+int prefill_tile_rows(const wz_moe_desc* d, int64_t T) {
+  const bool fits = int64_t(d->inter) * d->dim < (int64_t(1) << 30) &&
+                    wide_lds(std::max(d->dim, d->inter)) <= 160 * 1024;
+  return fits && d->act_scale_kind != WZ_SCALE_F32 && T >= 1024 && T * d->topk >= 32 * int64_t(d->n_experts) ? kPrefillWideRows : kPM;
+}
+
 // A dense MXFP4 linear in tiles: block b = (M-tile b / nblk, N-block b % nblk).
 // CHAIN: power-of-two activation scales (they ride in the MFMA with the e8m0
 // weight scales).
@@ -1053,12 +1336,15 @@ int launch_prefill_experts(const wz_moe_desc* d, const MoeWs& w, const void* x, 
   const bool cr = d->act_scale_kind != WZ_SCALE_F32;
   const bool cs = cr && d->shared_w_scale_kind == WZ_WSCALE_E8M0;
   const int Ti = int(T), dn13 = int(mt_dense * nb13d), dn2 = int(mt_dense * nb2d);
-  const dim3 blk(kPThreads), g13(unsigned(dn13 + mt_max * nb13)), g2(unsigned(dn2 + mt_max * nb2));
+  const dim3 blk(kPThreads);
   // routed block order (tile_order): 8 M-tiles x 8 N-blocks per group at T >= 1024,
   // where skewed batches give hot experts many M-tiles (T = 2048, calibrated skew:
   // 1327 -> 1250 us per layer); M-tile major below (T = 128: 341 vs 367 us)
   const bool grouped = T >= 1024;
   const int gm = grouped ? 8 : 1, gn13 = grouped ? 8 : nb13, gn2 = grouped ? 8 : nb2;
+  // wide routed tiles: the shared expert's dense blocks in a launch of their own
+  const bool wide = prefill_tile_rows(d, T) == kPrefillWideRows;
+  const dim3 g13(unsigned(dn13 + (wide ? 0 : mt_max * nb13))), g2(unsigned(dn2 + (wide ? 0 : mt_max * nb2)));
   if (only < 0 || only == WZ_STAGE_W13) {
     if (cr && cs) {
       WZ_LAUNCH("moe_w13", stream, (prefill_gemm_kernel<true, true, true>), g13, blk, 0, *d, w, Ti, nb13, nb13d, dn13, gm, gn13);
@@ -1069,6 +1355,8 @@ int launch_prefill_experts(const wz_moe_desc* d, const MoeWs& w, const void* x, 
                 dn13, gm, gn13);
     }
     if (int rc = check_launch("moe w13")) return rc;
+    if (wide)
+      if (int rc = launch_wide<true>(d, w, T, I / 128, stream)) return rc;
   }
   // the routed h rows are quantised in the w1/w3 epilogue; the shared rows here
   if (only < 0 || only == WZ_STAGE_HQUANT) {
@@ -1083,6 +1371,8 @@ int launch_prefill_experts(const wz_moe_desc* d, const MoeWs& w, const void* x, 
       WZ_LAUNCH("moe_w2", stream, (prefill_gemm_kernel<false, false, false>), g2, blk, 0, *d, w, Ti, nb2, nb2d, dn2, gm, gn2);
     }
     if (int rc = check_launch("moe w2")) return rc;
+    if (wide)
+      if (int rc = launch_wide<false>(d, w, T, (D + 255) / 256, stream)) return rc;
   }
   return WZ_OK;
 }
