@@ -151,6 +151,70 @@ __global__ __launch_bounds__(kGemmThreads) void grouped_fp4_kernel(const uint8_t
                                  WZ_WSCALE_E8M0, C + g * N, 1, N, K, 0, blockIdx.x * 16);
 }
 
+// The same products with K = 512 U (a wave's K quarter is U K-blocks).  The skinny body asks
+// memory 5 U times a wave (a tile, a scale byte per K-block and row, two pieces of the row and
+// its scale), most of them for a few bytes of many lines, and that issue rate bounds it: here
+// the row and its scales come into LDS once a workgroup, and a weight row's scales of the
+// quarter in 16-byte loads, U + U / 4 + 2 requests a wave at 59 registers (seven waves a SIMD)
+// instead of 150 (three).  Same products in the same order.  Six rows of 4096 x 4096 17.7 ->
+// 15.3 us, 3.5 TB/s; the weights through LDS in whole lines took 15.1, not worth their LDS.
+template <int U>
+__global__ __launch_bounds__(kGemmThreads) void grouped_fp4_row_kernel(const uint8_t* __restrict__ A,
+                                                                       const void* __restrict__ As, int act_kind,
+                                                                       const uint8_t* __restrict__ W,
+                                                                       const uint8_t* __restrict__ Ws,
+                                                                       uint16_t* __restrict__ C, int N) {
+  constexpr int K = 512 * U, KB = 4 * U;
+  __shared__ __align__(16) uint8_t a_l[K];
+  __shared__ uint32_t as_l[KB];  // e8m0 byte, or the float's bits
+  __shared__ float red[4][kWave][4];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int nl = lane & 15, g = lane >> 4;
+  const int64_t grp = blockIdx.y, row = grp * N + blockIdx.x * 16 + nl;
+  const uint8_t* const wr = W + row * (K / 2) + wave * (U * 64) + g * 16;
+  const uint8_t* const sr = Ws + row * (K / 32) + wave * (U * 4);
+  if (tid * 16 < K) *reinterpret_cast<v4i*>(a_l + tid * 16) = load16(A + grp * K + tid * 16);
+  if (tid < KB)
+    as_l[tid] = act_kind == WZ_SCALE_UE8M0 ? uint32_t(static_cast<const uint8_t*>(As)[grp * KB + tid])
+                                           : static_cast<const uint32_t*>(As)[grp * KB + tid];
+  v4i b[U], sd[U / 4];
+#pragma unroll
+  for (int u = 0; u < U; ++u) b[u] = load16(wr + u * 64);
+#pragma unroll
+  for (int u = 0; u < U / 4; ++u) sd[u] = load16(sr + u * 16);
+  __syncthreads();
+  const bool a_pow2 = act_kind != WZ_SCALE_F32;
+  v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int kb = wave * U + u;
+    AOp a = a_zero();
+    const v4i lo = *reinterpret_cast<const v4i*>(a_l + kb * 128 + g * 16);
+    const v4i hi = *reinterpret_cast<const v4i*>(a_l + kb * 128 + g * 16 + 64);
+    a.v = v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    const uint32_t s = as_l[kb];
+    if (act_kind == WZ_SCALE_UE8M0)
+      a.se8 = int(s);
+    else if (act_kind == WZ_SCALE_UE8M0_F32)
+      a.se8 = int((s >> 23) & 0xFFu);
+    else
+      a.sf = __uint_as_float(s);
+    const v8i bv = {b[u][0], b[u][1], b[u][2], b[u][3], 0, 0, 0, 0};
+    mma_step<kFmtFp8, kFmtFp4>(acc, a, bv, int((uint32_t(sd[u / 4][u & 3]) >> (8 * g)) & 0xFFu), 1.0f, a_pow2, true,
+                               lane);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) red[wave][lane][i] = acc[i];
+  __syncthreads();
+  if (tid < 16) {  // row 0 of the tile: element 0 of lane group 0; partials in wave order
+    float v = red[0][tid][0];
+    v += red[1][tid][0];
+    v += red[2][tid][0];
+    v += red[3][tid][0];
+    C[grp * N + blockIdx.x * 16 + tid] = f32_to_bf16(v);
+  }
+}
+
 template <int WF, bool A_BF16>
 static int launch_skinny(const void* A, const void* As, int act_kind, const void* W, const void* Ws,
                          int w_kind, void* C, int64_t M, int64_t N, int64_t K, hipStream_t stream,
@@ -263,7 +327,17 @@ extern "C" int wz_grouped_fp4_gemm(const void* a_e4m3, const void* a_s, const vo
   const uint8_t* ws = static_cast<const uint8_t*>(w_s_e8m0);
   uint16_t* c = static_cast<uint16_t*>(c_bf16);
   const int u = skinny_unroll(K);
-  if (u == 8) {
+  // the row kernel reads 16 bytes at a time; other K and unaligned operands take the skinny body
+  const bool vec = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(w) |
+                     reinterpret_cast<uintptr_t>(ws)) & 15) == 0 &&
+                   (act_scale_kind == WZ_SCALE_UE8M0 || (reinterpret_cast<uintptr_t>(a_s) & 3) == 0);
+  if (vec && K == 4096) {
+    WZ_LAUNCH("grouped_fp4_gemm", stream, grouped_fp4_row_kernel<8>, grid, dim3(kGemmThreads), 0, a, a_s,
+              act_scale_kind, w, ws, c, int(N));
+  } else if (vec && K == 2048) {
+    WZ_LAUNCH("grouped_fp4_gemm", stream, grouped_fp4_row_kernel<4>, grid, dim3(kGemmThreads), 0, a, a_s,
+              act_scale_kind, w, ws, c, int(N));
+  } else if (u == 8) {
     WZ_LAUNCH("grouped_fp4_gemm", stream, grouped_fp4_kernel<8>, grid, dim3(kGemmThreads), 0, a, a_s, act_scale_kind,
               w, ws, c, int(N), int(K));
   } else if (u == 4) {
