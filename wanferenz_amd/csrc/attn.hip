@@ -31,12 +31,12 @@ __host__ __device__ constexpr int64_t attn_part_floats(int d) { return 128 + 64 
 
 // LDS image of one block of 64 KV rows, row-major, no padding.  The 16-byte
 // chunks of row r sit XOR-swizzled (chunk c at slot c ^ swz(r)) so that both
-// read patterns are free of bank conflicts.  A 16-byte read of one chunk of
+// read patterns spread over the banks.  A 16-byte read of one chunk of
 // 16 rows (the K operand of S^T) is served in passes of 16 lanes that mix rows
 // 0-3 and 12-15 of one lane group with rows 4-11 of the next, whose chunk is
 // the neighbour: the slots of rows 0-3 and 12-15 are closed under ^ 1, so the
-// passes' slots are distinct (without that, every pass took two turns: 45 % of
-// the LDS cycles).  The transpose reads of V take two adjacent chunks of 8
+// passes' slots are distinct (conflicts took 44 % of the LDS cycles without
+// that, 30 % with it; P's 8-byte writes and the transpose reads are the rest).  The transpose reads of V take two adjacent chunks of 8
 // consecutive rows, which have distinct slot pairs.
 template <int D>
 struct KsLayout {
