@@ -9,6 +9,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+
 #include "wanferenz_amd.h"
 
 namespace wz {
@@ -286,6 +288,16 @@ namespace wz {
 int set_error(int code, const char* fmt, ...);
 int check_launch(const char* what);
 int cu_count();
+constexpr int kMaxDevices = 64;  // devices of a process that per-device state is kept for
+// Dynamic LDS granted to one kernel (a static of its launch code), per device.
+struct LdsGrant {
+  std::atomic<int> bytes[kMaxDevices];
+};
+int allow_lds_of(const char* what, const void* kernel, size_t bytes, LdsGrant& grant);
+template <typename F>
+int allow_lds(const char* what, F* kernel, size_t bytes, LdsGrant& grant) {
+  return allow_lds_of(what, reinterpret_cast<const void*>(kernel), bytes, grant);
+}
 int prof_pre(hipStream_t s, hipEvent_t* start, hipEvent_t* stop);
 void prof_post(int slot, const char* name);
 }  // namespace wz

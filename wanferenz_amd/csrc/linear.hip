@@ -746,18 +746,7 @@ static size_t gemv1_dyn_bytes(bool qa, int64_t M, int64_t K, int W, int RT) {
   return qa ? red : std::max(gemv1_lds_bytes(M, K), red);
 }
 
-// LDS a workgroup may hold on gfx950 (160 KB); dynamic LDS past 64 KB is
-// requested per kernel once (hipFuncAttributeMaxDynamicSharedMemorySize).
-constexpr size_t kLdsMax = 160 * 1024;
-template <typename F>
-static int allow_lds(F* kernel, size_t bytes, int& granted) {
-  if (bytes <= 64 * 1024 || int(bytes) <= granted) return 0;
-  if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                          int(bytes)) != hipSuccess)
-    return set_error(WZ_ELAUNCH, "fp8 gemv: %zu bytes of LDS refused", bytes);
-  granted = int(bytes);
-  return 0;
-}
+constexpr size_t kLdsMax = 160 * 1024;  // LDS a workgroup may hold on gfx950
 
 template <int W, int NKB, int NB, int MINW, bool XF, bool QA>
 static int launch_gemv(const void* x, const void* xs, int a_kind, const uint8_t* w, const void* w_s, int w_kind,
@@ -920,8 +909,8 @@ static int launch_gemv1_rt(const void* x, const void* xs, int a_kind, const uint
   const size_t lds = gemv1_dyn_bytes(QA, M, K, W, RT);
 #define WZ_GV1(AP, BP)                                                                                        \
   do {                                                                                                          \
-    static int granted = 0;                                                                                     \
-    if (int rc = allow_lds(fp8_gemv1_kernel<W, NKB, XP, QA, AP, BP, false, RT>, lds, granted)) return rc;          \
+    static LdsGrant grant;                                                                                      \
+    if (int rc = allow_lds("fp8 gemv", fp8_gemv1_kernel<W, NKB, XP, QA, AP, BP, false, RT>, lds, grant)) return rc;\
     WZ_LAUNCH("fp8_gemv1", stream, (fp8_gemv1_kernel<W, NKB, XP, QA, AP, BP, false, RT>), grid, block, lds, x, xs,  \
               a_kind, w, w_s, res, y, y_hi, int(n_split), int(M), int(N), int(K), nullptr, 0.0f, nullptr, nullptr, 1); \
   } while (0)
@@ -958,8 +947,8 @@ static int launch_gemv_mt(const void* xq, const void* xs, int a_kind, const uint
   const size_t lds = gemv1_dyn_bytes(true, M, K, W, RT);
 #define WZ_GVM(AP, BP)                                                                                        \
   do {                                                                                                          \
-    static int granted = 0;                                                                                     \
-    if (int rc = allow_lds(fp8_gemv1_kernel<W, NKB, 1, true, AP, BP, false, RT>, lds, granted)) return rc;         \
+    static LdsGrant grant;                                                                                      \
+    if (int rc = allow_lds("fp8 gemv", fp8_gemv1_kernel<W, NKB, 1, true, AP, BP, false, RT>, lds, grant)) return rc;\
     WZ_LAUNCH("fp8_gemv_mt", stream, (fp8_gemv1_kernel<W, NKB, 1, true, AP, BP, false, RT>), grid, block, lds, xq,   \
               xs, a_kind, w, w_s, res, y, y_hi, int(n_split), int(M), int(N), int(K), nullptr, 0.0f, nullptr,     \
               nullptr, n_mt);                                                                                   \
@@ -1352,8 +1341,8 @@ static int launch_norm_gemv1(const void* x, const uint16_t* b, const float* nw, 
   const bool bp = w_kind == WZ_WSCALE_E8M0;
 #define WZ_NG1(AP, BP)                                                                                          \
   do {                                                                                                          \
-    static int granted = 0;                                                                                     \
-    if (int rc = allow_lds(fp8_gemv1_kernel<W, NKB, 1, false, AP, BP, true, 1>, lds, granted)) return rc;             \
+    static LdsGrant grant;                                                                                      \
+    if (int rc = allow_lds("fp8 gemv", fp8_gemv1_kernel<W, NKB, 1, false, AP, BP, true, 1>, lds, grant)) return rc;\
     WZ_LAUNCH("fp8_norm_gemv1", stream, (fp8_gemv1_kernel<W, NKB, 1, false, AP, BP, true, 1>), grid, block, lds, x, nullptr, 0, \
               w, w_s, nullptr, y, y_hi, int(n_split), int(M), int(N), int(K), nw, eps, b, hsum, 1);            \
   } while (0)

@@ -29,7 +29,6 @@
 #include "mfma_ops.h"
 
 #include <algorithm>
-#include <atomic>
 
 namespace wz {
 
@@ -368,13 +367,8 @@ static size_t tile_lds(int64_t K, bool a_pow2) {
 template <class C, int WF, bool AP2, bool BP2, bool SL1>
 static int launch_tile(const char* name, TileArgs p, hipStream_t stream) {
   const size_t lds = tile_lds<C, WF>(p.K, AP2);
-  static std::atomic<int> granted{0};
-  if (int(lds) > granted.load(std::memory_order_relaxed)) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(tile_gemm_kernel<C, WF, AP2, BP2, SL1>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)) != hipSuccess)
-      return set_error(WZ_ELAUNCH, "%s: %zu bytes of LDS refused", name, lds);
-    granted.store(int(lds), std::memory_order_relaxed);
-  }
+  static LdsGrant grant;
+  if (int rc = allow_lds(name, tile_gemm_kernel<C, WF, AP2, BP2, SL1>, lds, grant)) return rc;
   p.n_mt = (p.M + C::BM - 1) / C::BM;
   p.n_nb = (p.N + C::BN - 1) / C::BN;
   WZ_LAUNCH(name, stream, (tile_gemm_kernel<C, WF, AP2, BP2, SL1>), dim3(unsigned(p.n_mt * p.n_nb)), dim3(C::NT), lds,

@@ -770,7 +770,6 @@ namespace wz {
 
 static __device__ __align__(256) uint8_t scratch[WZ_MOE_NOALLOC_SCRATCH_BYTES];
 
-constexpr int kMaxDevices = 64;
 static void* g_scratch_ptr[kMaxDevices];
 static std::once_flag g_scratch_once[kMaxDevices];
 static int g_scratch_rc[kMaxDevices];

@@ -22,7 +22,6 @@
 #include "moe_common.h"
 
 #include <algorithm>
-#include <atomic>
 #include <type_traits>
 
 namespace wz {
@@ -1276,13 +1275,8 @@ __global__ __launch_bounds__(kWideThreads, 4) void prefill_wide_kernel(wz_moe_de
 template <bool W13>
 static int launch_wide(const wz_moe_desc* d, const MoeWs& w, int64_t T, int nblk, hipStream_t stream) {
   const size_t lds = wide_lds(W13 ? d->dim : d->inter);
-  static std::atomic<int> granted{0};
-  if (int(lds) > granted.load(std::memory_order_relaxed)) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_wide_kernel<W13>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)) != hipSuccess)
-      return set_error(WZ_ELAUNCH, "moe prefill: %zu bytes of LDS refused", lds);
-    granted.store(int(lds), std::memory_order_relaxed);
-  }
+  static LdsGrant grant;
+  if (int rc = allow_lds("moe prefill", prefill_wide_kernel<W13>, lds, grant)) return rc;
   const int64_t P = T * d->topk, E = d->n_experts;
   const int64_t mt_max = P / kPrefillWideRows + std::min(P, E) + 1;
   WZ_LAUNCH(W13 ? "moe_w13" : "moe_w2", stream, prefill_wide_kernel<W13>, dim3(unsigned(mt_max * nblk)),
