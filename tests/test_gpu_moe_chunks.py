@@ -67,3 +67,25 @@ def test_wide_tiles_equal_narrow_ones(gpu, E, T, skew):
         ws = torch.empty(moe.workspace_bytes(n), dtype=torch.uint8, device=gpu)
         for a, b in zip((y, w, i), _run(moe, x[at:at + n].contiguous(), ws)):
             assert torch.equal(a[at:at + n], b)
+
+
+def test_captured_long_prompt(gpu):
+    """The larger workspace of a captured long prompt belongs to the graph: replays, with eager
+    calls of other lengths between them, give the eager bits."""
+    from tests.test_gpu_moe import upload_case
+
+    T = 2731 + 16
+    case = dataclasses.replace(CASES["top6_t8"], name="captured_chunk", dim=256, inter=128, n_experts=128, T=T)
+    inp = make_inputs(case)
+    moe = upload_case(case, inp, gpu)
+    x = bf16_tensor(inp.x, gpu)
+    y = moe.forward(x)
+    moe.reserve(T)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = moe.forward(x)
+    for n in (8, 200, T):
+        g.replay()
+        assert torch.equal(out, y)
+        assert torch.equal(moe.forward(x[:n].contiguous()), y[:n])
+        out.zero_()

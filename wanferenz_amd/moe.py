@@ -6,8 +6,9 @@ Two ways in:
   (w13 ``[E, 2I, D/2]`` packed e2m1 + ``[E, 2I, D/32]`` e8m0, w2 ``[E, D, I/2]``
   + ``[E, D, I/32]``, the bank layout of wanferenz/kernels/fp4_grouped.py:142-188)
   with an FP8 shared expert and a bf16 gate.  ``forward(x, input_ids)`` is one
-  stream-ordered sequence of launches with no host sync and no allocation
-  besides its output, so a decode step can be captured in a HIP graph.
+  stream-ordered sequence of launches with no host sync and, up to one chunk of
+  16384 routed pairs, no allocation besides its output, so a decode step can be
+  captured in a HIP graph.
 * :func:`install` — replaces ``MoE.forward`` of a loaded reference model module
   at class level, following the reference's install protocol
   (fp4_grouped.py:339-351): the previous forward is kept in ``_REF_FORWARD``,
@@ -31,6 +32,10 @@ import torch
 
 from . import _native as N
 from . import kernels
+
+# Routed pairs of a chunk that every layer size runs (kMaxPairs, csrc/moe_common.h): the
+# workspace a layer holds is never larger than that of one such chunk.
+CHUNK_PAIRS = 16384
 
 SCORE_FUNCS = {"softmax": N.WZ_SCORE_SOFTMAX, "sigmoid": N.WZ_SCORE_SIGMOID,
                "sqrtsoftplus": N.WZ_SCORE_SQRTSOFTPLUS}
@@ -277,13 +282,22 @@ class HipMoE:
         return int(N.lib().wz_moe_workspace_bytes(ctypes.byref(self.desc), T))
 
     def reserve(self, T: int):
-        """Allocate scratch for up to T tokens (outside any graph capture)."""
+        """Allocate scratch that serves calls of up to T tokens (outside any graph capture).
+
+        The layer holds at most the scratch of one chunk of ``CHUNK_PAIRS`` routed pairs
+        (0.3 GB at V4 sizes), whatever T: layers run one after another, so what a longer
+        prompt can use beyond that is taken for the call (:meth:`_prompt_ws`)."""
         if T <= self._ws_tokens and self._ws is not None:
             return
-        nbytes = max(self.workspace_bytes(T), 256)
-        self._ws = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
-        N.call("wz_moe_workspace_init", self._ws.data_ptr(), nbytes, N.stream_handle(self.device))
+        nbytes = max(self.workspace_bytes(min(T, CHUNK_PAIRS // self.cfg.topk)), 256)
+        if self._ws is None or nbytes > self._ws.numel():
+            self._ws = self._new_ws(nbytes)
         self._ws_tokens = T
+
+    def _new_ws(self, nbytes: int) -> torch.Tensor:
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
+        N.call("wz_moe_workspace_init", ws.data_ptr(), nbytes, N.stream_handle(self.device))
+        return ws
 
     def _ws_for(self, T: int):
         if T > self._ws_tokens:
@@ -293,6 +307,22 @@ class HipMoE:
                     "inside graph capture; call reserve() before capturing")
             self.reserve(T)
         return self._ws
+
+    def _prompt_ws(self, T: int):
+        """Scratch of a forward of T tokens.  Past CHUNK_PAIRS routed pairs a layer of many
+        experts runs larger chunks where the scratch holds them; that scratch comes from
+        torch's allocator for the one call (on the current stream, so the next layer's call
+        gets the same memory), and where there is none the layer's own serves, in more chunks."""
+        ws = self._ws_for(T)
+        if T * self.cfg.topk <= CHUNK_PAIRS:
+            return ws
+        nbytes = self.workspace_bytes(T)
+        if nbytes <= ws.numel():
+            return ws
+        try:
+            return self._new_ws(nbytes)
+        except torch.OutOfMemoryError:
+            return ws
 
     # -- compute -------------------------------------------------------------
     def _tokens(self, x: torch.Tensor) -> torch.Tensor:
@@ -347,7 +377,7 @@ class HipMoE:
             self._check_out(routing_out[0], (T, k), torch.float32, "routing weights")
             self._check_out(routing_out[1], (T, k), torch.int64, "routing indices")
             wp, ip = routing_out[0].data_ptr(), routing_out[1].data_ptr()
-        ws = self._ws_for(T)
+        ws = self._prompt_ws(T)
         N.call("wz_moe_forward", ctypes.byref(self.desc), xv.data_ptr(), _ptr(ids), T, y.data_ptr(), wp, ip,
                ws.data_ptr(), ws.numel(), N.stream_handle(self.device))
         return y.view(x.shape)
@@ -396,7 +426,7 @@ class HipMoE:
         """
         xv = self._tokens(x)
         T = xv.size(0)
-        if T > self._ws_tokens or T * self.cfg.topk > 16384:
+        if T > self._ws_tokens or T * self.cfg.topk > CHUNK_PAIRS:
             raise RuntimeError("HipMoE.replay_stage: no preceding single-chunk forward with this many tokens")
         self._check_out(out, (T, self.cfg.dim), torch.bfloat16, "out")
         ids = self._ids(input_ids, T)
