@@ -84,7 +84,7 @@ def test_captured_long_prompt(gpu):
     g = torch.cuda.CUDAGraph()
     with torch.cuda.graph(g):
         out = moe.forward(x)
-    for n in (8, 200, T):
+    for n in (32, 200, T):
         g.replay()
         assert torch.equal(out, y)
         assert torch.equal(moe.forward(x[:n].contiguous()), y[:n])

@@ -348,8 +348,9 @@ __global__ __launch_bounds__(C::NT, C::OCC * C::W / 4) void tile_gemm_kernel(Til
 // ------------------------------------------------------------------ host ----
 
 // A tile shape and its cost: t1 is the time of a grid of at most one workgroup per CU, t2 that
-// of a full round of PER_CU workgroups on every CU (us at K = 4096, measured; the ratios hold
-// at K = 1024 ... 8192).
+// of a full round of PER_CU workgroups on every CU (us at K = 4096, power-of-two activation
+// scales, measured).  Over 17 ... 2048 rows, K = 1024 ... 12288 and both scale kinds the shape of
+// the lowest cost takes 0.3 to 1.1 % more time than the fastest on average, 28 % at worst.
 template <class C_, int PER_CU_, int T1_, int T2_>
 struct TileShape {
   using C = C_;
@@ -376,40 +377,36 @@ static int launch_tile(const char* name, TileArgs p, hipStream_t stream) {
   return check_launch(name);
 }
 
-template <class C, int WF, bool SL1>
-static int launch_tile_kinds(const char* name, const TileArgs& p, bool a_pow2, bool b_pow2, hipStream_t stream) {
-  if constexpr (SL1) {
-    return launch_tile<C, WF, true, true, true>(name, p, stream);
-  } else {
-    if (WF == kWRowsFp4)  // its scales are e8m0: BP2
-      return a_pow2 ? launch_tile<C, WF, true, true, false>(name, p, stream)
-                    : launch_tile<C, WF, false, true, false>(name, p, stream);
-    if (a_pow2)
-      return b_pow2 ? launch_tile<C, WF, true, true, false>(name, p, stream)
-                    : launch_tile<C, WF, true, WF == kWRowsFp4, false>(name, p, stream);
-    return b_pow2 ? launch_tile<C, WF, false, true, false>(name, p, stream)
-                  : launch_tile<C, WF, false, WF == kWRowsFp4, false>(name, p, stream);
-  }
+template <class C, int WF, bool AP2, bool SL1>
+static int launch_tile_kinds(const char* name, const TileArgs& p, bool b_pow2, hipStream_t stream) {
+  if constexpr (SL1 || WF == kWRowsFp4)  // fp4 scales are e8m0
+    return launch_tile<C, WF, AP2, true, SL1>(name, p, stream);
+  else
+    return b_pow2 ? launch_tile<C, WF, AP2, true, false>(name, p, stream)
+                  : launch_tile<C, WF, AP2, false, false>(name, p, stream);
 }
 
-// Time of the whole grid in rounds of the shape (infinite where its LDS does not fit).
+// Time of the whole grid in rounds of the shape (infinite where its LDS does not fit).  A CU holds
+// PER_CU workgroups, or one where the K range's scales (four bytes a row and K-block for float
+// ones) leave room for no more: a round of those costs T1.
 template <class Sh, int WF>
 static double shape_cost(const TileArgs& p, bool a_pow2) {
   using C = typename Sh::C;
-  if (tile_lds<C, WF>(p.K, a_pow2) > kTileLds) return 1e30;
-  const int64_t cus = cu_count();
+  const size_t lds = tile_lds<C, WF>(p.K, a_pow2);
+  if (lds > kTileLds) return 1e30;
+  const int64_t cus = cu_count(), held = std::min<int64_t>(Sh::PER_CU, kTileLds / lds);
   const int64_t blocks = int64_t((p.M + C::BM - 1) / C::BM) * ((p.N + C::BN - 1) / C::BN);
   if (blocks <= cus) return Sh::T1;
-  const int64_t round = cus * Sh::PER_CU;
-  return double((blocks + round - 1) / round) * Sh::T2;
+  const int64_t round = cus * held;
+  return double((blocks + round - 1) / round) * (held == Sh::PER_CU ? Sh::T2 : Sh::T1);
 }
 
-template <int WF, bool SL1, class... Shapes>
-static int launch_best(const char* name, const TileArgs& p, bool a_pow2, bool b_pow2, hipStream_t stream) {
-  const double cost[] = {shape_cost<Shapes, WF>(p, a_pow2)...};
+template <int WF, bool AP2, bool SL1, class... Shapes>
+static int launch_best(const char* name, const TileArgs& p, bool b_pow2, hipStream_t stream) {
+  const double cost[] = {shape_cost<Shapes, WF>(p, AP2)...};
   const int best = int(std::min_element(cost, cost + sizeof...(Shapes)) - cost);
   int i = 0, rc = WZ_OK;
-  (void)((i++ == best ? (rc = launch_tile_kinds<typename Shapes::C, WF, SL1>(name, p, a_pow2, b_pow2, stream), true)
+  (void)((i++ == best ? (rc = launch_tile_kinds<typename Shapes::C, WF, AP2, SL1>(name, p, b_pow2, stream), true)
                       : false) ||
          ...);
   return rc;
@@ -428,6 +425,8 @@ static int launch_best(const char* name, const TileArgs& p, bool a_pow2, bool b_
 // fp8 100 x 4096 x 4096 33 -> 11.4 us, fp4 333 x 2048 x 4096 59 -> 12.5 us.
 using Sh32 = TileShape<TileCfg<1, 1, 2, 2, 1, 8, 2>, 1, 105, 105>;
 using Sh32w = TileShape<TileCfg<1, 2, 2, 2, 2, 2, 2>, 2, 122, 144>;
+// 64 x 64 is one of the choices where float scales leave one 32 x 64 workgroup a CU: 200 x 4096 x
+// 8192 in 27.5 us against 45.0, 512 x 2048 x 12288 in 37.0 against 63.4.
 using Sh64 = TileShape<TileCfg<1, 2, 4, 2, 2, 2, 2>, 1, 147, 153>;
 using Sh64w = TileShape<TileCfg<1, 4, 4, 2, 2, 1, 2>, 2, 184, 297>;
 using Sh128 = TileShape<TileCfg<2, 4, 4, 2, 1, 1, 2>, 2, 270, 486>;
@@ -477,8 +476,9 @@ int launch_tile_gemm(const uint8_t* xq, const void* xs, int a_kind, const uint8_
   p.order = SliceOrder{slice, 1};
   p.vec = aligned16(y) && aligned16(y_hi) && aligned16(res) && n_split % 8 == 0;
   if (slice == 1 && ap && bp)
-    return launch_best<kWPacked, true, Sh32, Sh32w, Sh64, Sh64w, Sh128, Sh256>("fp8_tile_gemm", p, ap, bp, stream);
-  return launch_best<kWPacked, false, Sh32, Sh32w, Sh64, Sh64w, Sh128>("fp8_tile_gemm", p, ap, bp, stream);
+    return launch_best<kWPacked, true, true, Sh32, Sh32w, Sh64w, Sh128, Sh256>("fp8_tile_gemm", p, bp, stream);
+  if (ap) return launch_best<kWPacked, true, false, Sh32, Sh32w, Sh64w, Sh128>("fp8_tile_gemm", p, bp, stream);
+  return launch_best<kWPacked, false, false, Sh32, Sh32w, Sh64, Sh64w, Sh128>("fp8_tile_gemm", p, bp, stream);
 }
 
 // Row-major weights (e4m3, or e2m1 with fp4) in skinny_gemm_kernel's summation order.  Served where the
@@ -506,8 +506,11 @@ int launch_tile_rows(const char* name, const uint8_t* a, const void* a_s, int a_
   p.K = int(K);
   p.order = SliceOrder{int(K / 128), 4};
   p.vec = aligned16(c);
-  if (fp4) return launch_best<kWRowsFp4, false, Sf32, Sf32w, Sf64, Sf64w, Sf128>(name, p, ap, bp, stream);
-  return launch_best<kWRows, false, Sh32, Sh32w, Sh64, Sh64w, Sh128>(name, p, ap, bp, stream);
+  if (fp4)
+    return ap ? launch_best<kWRowsFp4, true, false, Sf32, Sf32w, Sf64, Sf64w, Sf128>(name, p, bp, stream)
+              : launch_best<kWRowsFp4, false, false, Sf32, Sf32w, Sf64, Sf64w, Sf128>(name, p, bp, stream);
+  return ap ? launch_best<kWRows, true, false, Sh32, Sh32w, Sh64w, Sh128>(name, p, bp, stream)
+            : launch_best<kWRows, false, false, Sh32, Sh32w, Sh64, Sh64w, Sh128>(name, p, bp, stream);
 }
 
 }  // namespace wz
