@@ -67,3 +67,20 @@ F32, E8 = N.WZ_SCALE_F32, N.WZ_SCALE_UE8M0
 def test_choice_counts_resident_workgroups(tmp_path, call, tile):
     _, got = selected(tmp_path, [call])
     assert [g[len("wz::TileCfg<"):].startswith(tile) for g in got] == [True], got
+
+
+# (call, served by the skinny kernel): up to 32 rows of a K of up to 2048, and up to 28 of MXFP4 at any
+# K, where both scales are powers of two and N / 16 workgroups fit the 256 CUs; 16 rows otherwise
+@pytest.mark.parametrize("call,skinny", [
+    (fp4_rows(16, 32768, 1024, F32), True), (fp4_rows(17, 2048, 4096, E8), True), (fp4_rows(28, 4096, 4096, E8), True),
+    (fp4_rows(29, 4096, 4096, E8), False), (fp4_rows(17, 4112, 4096, E8), False), (fp4_rows(17, 2048, 4096, F32), False),
+    (fp4_rows(28, 16, 12288, N.WZ_SCALE_UE8M0_F32), True), (fp4_rows(32, 4096, 2048, E8), True),
+    (fp8_rows(16, 32768, 1024, True, F32), True), (fp8_rows(32, 4096, 2048, False, E8), True),
+    (fp8_rows(33, 4096, 2048, False, E8), False), (fp8_rows(17, 4096, 2176, False, E8), False),
+    (fp8_rows(17, 4096, 2048, True, E8), False), (fp8_rows(17, 4096, 2048, False, F32), False),
+    (fp8_rows(17, 4112, 1024, False, E8), False),
+])
+def test_rows_of_the_skinny_kernel(tmp_path, call, skinny):
+    _, events = record(tmp_path, [call])
+    (name,) = [e["name"] for e in events if e["kind"] == "launch"]
+    assert ("skinny_gemm_kernel" in name) == skinny, name

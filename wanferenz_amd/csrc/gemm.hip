@@ -20,11 +20,21 @@ namespace wz {
 
 constexpr int kGemmThreads = 256;
 
-// Above this many rows the tile GEMM (linear_gemm.hip; the same summation order, so the same
-// bits) takes over: one M-tile of 16 is all padding-free MFMA work of a weight stream that is
-// read once, from two on the skinny kernel's re-reads of the rows by every 16 columns cost more
-// than staging both operands (17 x 4096 x 4096 fp8 11.9 -> 9.1 us, fp4 10.7 -> 9.7 us).
-constexpr int kSkinnyMaxM = 16;
+// Rows up to which the skinny kernel serves; above, the tile GEMM (linear_gemm.hip; the same
+// summation order, so the same bits).  One M-tile of 16 is padding-free MFMA work of a weight
+// stream that is read once; from two on the skinny kernel's re-reads of the rows by every 16
+// columns cost more than staging both operands, except where both scales ride in the MFMA and a
+// workgroup per 16 columns fits the CUs at once: there its wider weight loads and four K quarters
+// win up to 32 rows of a K of up to 2048 (skinny / tile us, e4m3 20 x 4096 x 2048 5.6 / 6.2, 32 x
+// 4096 x 1024 4.1 / 4.6, MXFP4 31 x 4096 x 1024 3.9 / 4.3) and, for MXFP4 weights, up to 28 rows of
+// a longer one (17 x 2048 x 4096 7.4 / 8.8, 28 rows 8.6 / 8.8, 32 rows 9.0 / 8.8; e4m3 at K = 4096
+// 17 rows 8.4 / 8.4).  Wider
+// N and float scales go the other way from 17 rows on (17 x 32768 x 1024 e4m3 14.8 / 9.2, MXFP4
+// 12.1 / 6.0; 17 x 4096 x 4096 with float scales 16.2 / 9.3).
+static int64_t skinny_max_rows(bool fp4, bool pow2, int64_t N, int64_t K) {
+  if (!pow2 || N / 16 > cu_count()) return 16;
+  return K <= 2048 ? 32 : fp4 ? 28 : 16;
+}
 bool tile_rows_fits(const void* a, const void* w, const void* w_s, bool fp4, int64_t M, int64_t N, int64_t K);
 int launch_tile_rows(const char* name, const uint8_t* a, const void* a_s, int a_kind, const uint8_t* w,
                      const void* w_s, int w_kind, bool fp4, uint16_t* c, int64_t M, int64_t N, int64_t K,
@@ -272,7 +282,8 @@ extern "C" int wz_fp8_gemm(const void* a_e4m3, const void* a_s, const void* w_e4
     return set_error(WZ_EINVAL, "fp8_gemm: bad scale kinds %d/%d", act_scale_kind, w_scale_kind);
   if (M && (!a_e4m3 || !a_s || !w_e4m3 || !w_s || !c_bf16))
     return set_error(WZ_EINVAL, "fp8_gemm: null pointer");
-  if (M > kSkinnyMaxM && tile_rows_fits(a_e4m3, w_e4m3, w_s, false, M, N, K))
+  const bool pow2 = act_scale_kind != WZ_SCALE_F32 && w_scale_kind == WZ_WSCALE_E8M0;
+  if (M > skinny_max_rows(false, pow2, N, K) && tile_rows_fits(a_e4m3, w_e4m3, w_s, false, M, N, K))
     return launch_tile_rows("fp8_gemm", static_cast<const uint8_t*>(a_e4m3), a_s, act_scale_kind,
                             static_cast<const uint8_t*>(w_e4m3), w_s, w_scale_kind, false,
                             static_cast<uint16_t*>(c_bf16), M, N, K, stream);
@@ -302,7 +313,8 @@ extern "C" int wz_fp4_gemm(const void* a_e4m3, const void* a_s, const void* w_fp
     return set_error(WZ_EINVAL, "fp4_gemm: bad scale kind %d", act_scale_kind);
   if (M && (!a_e4m3 || !a_s || !w_fp4x2 || !w_s_e8m0 || !c_bf16))
     return set_error(WZ_EINVAL, "fp4_gemm: null pointer");
-  if (M > kSkinnyMaxM && tile_rows_fits(a_e4m3, w_fp4x2, w_s_e8m0, true, M, N, K))
+  if (M > skinny_max_rows(true, act_scale_kind != WZ_SCALE_F32, N, K) &&
+      tile_rows_fits(a_e4m3, w_fp4x2, w_s_e8m0, true, M, N, K))
     return launch_tile_rows("fp4_gemm", static_cast<const uint8_t*>(a_e4m3), a_s, act_scale_kind,
                             static_cast<const uint8_t*>(w_fp4x2), w_s_e8m0, WZ_WSCALE_E8M0, true,
                             static_cast<uint16_t*>(c_bf16), M, N, K, stream);
