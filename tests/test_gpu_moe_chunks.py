@@ -48,14 +48,18 @@ def test_large_chunks_equal_small_ones(gpu, E, T):
         assert torch.equal(big[0][t:t + 32], moe.forward(x[t:t + 32].contiguous()))
 
 
-# the wide routed tiles (1024 tokens and 32 pair rows an expert on) against calls below them, whose
-# rows are in 64-row tiles: a partial last N-block of w2 (640 columns), five K-blocks (a ragged
-# group of scales), experts of many tiles and of few rows, a skewed selection with empty experts
-@pytest.mark.parametrize("E,T,skew", [(5, 1024, 0.0), (40, 1111, 0.0), (64, 1500, 0.05), (17, 2100, 1.0)])
+# the wide routed tiles against calls of 700 tokens, whose rows are in 64-row tiles: a partial last
+# N-block of w2 (640 columns), five K-blocks (a ragged group of scales), experts of many tiles and of
+# few rows, a skewed selection with empty experts (test_moe_routes.py: each case takes wide tiles)
+WIDE = dict(dim=640, inter=384, topk=2)
+WIDE_CASES = [(5, 5200, 0.0), (40, 3011, 0.0), (64, 1555, 0.05), (17, 4500, 1.0)]
+
+
+@pytest.mark.parametrize("E,T,skew", WIDE_CASES)
 def test_wide_tiles_equal_narrow_ones(gpu, E, T, skew):
     from tests.test_gpu_moe import upload_case
 
-    case = dataclasses.replace(CASES["top6_t8"], name=f"wide_e{E}_t{T}", dim=640, inter=384, n_experts=E, topk=2, T=T)
+    case = dataclasses.replace(CASES["top6_t8"], name=f"wide_e{E}_t{T}", n_experts=E, T=T, **WIDE)
     inp = make_inputs(case)
     moe = upload_case(case, inp, gpu)
     if skew:

@@ -1284,15 +1284,24 @@ static int launch_wide(const wz_moe_desc* d, const MoeWs& w, int64_t T, int nblk
   return check_launch(W13 ? "moe w13" : "moe w2");
 }
 
-// Pair rows per M-tile of a prefill of T tokens.  Wide tiles from 1024 tokens and 32 rows an
-// expert on, where both sides cross (256 experts of 4096 x 2048, us a layer, 64-row against
-// wide tiles): 16 rows 640 / 683, 24 rows 734 / 734, 35 rows 804 / 785, 48 rows 882 / 850,
-// 141 rows 1868 / 1589.  With fewer rows the launch streams weights from memory, and the
-// 64-row tiles keep three K-blocks in flight.
+// Pair rows per M-tile of a prefill of T tokens.  Wide tiles from 1024 tokens on, where both of
+// these hold (us a layer, 64-row against wide tiles):
+//  * rows an expert: below, the launch streams weights from memory, and the 64-row tiles keep
+//    three K-blocks in flight.  From 32 with I of 2048 or more (256 experts of 4096 x 2048:
+//    24 rows 734 / 734, 35 rows 804 / 785, 48 rows 882 / 850, 141 rows 1868 / 1589); from 48
+//    with a smaller I, where w2 has few K-blocks to fill and drain around (160 of 5120 x 1536:
+//    38 rows 547 / 577, 45 rows 590 / 599, 56 rows 658 / 632; 256 of 2048 x 512: 32 rows 183 /
+//    196, 64 rows 248 / 227);
+//  * a w1/w3 workgroup for each of 256 CUs: fewer, longer workgroups leave the others idle (8
+//    experts of 1024 x 512, top-2: 1500 tokens 75 / 88, 3000 tokens 95 / 98, 4096 tokens 124 /
+//    112; 16 of 512 x 256, top-2: 2048 tokens 67 / 78, 8192 tokens 130 / 119).
 int prefill_tile_rows(const wz_moe_desc* d, int64_t T) {
   const bool fits = int64_t(d->inter) * d->dim < (int64_t(1) << 30) &&
                     wide_lds(std::max(d->dim, d->inter)) <= 160 * 1024;
-  return fits && d->act_scale_kind != WZ_SCALE_F32 && T >= 1024 && T * d->topk >= 32 * int64_t(d->n_experts) ? kPrefillWideRows : kPM;
+  if (!fits || d->act_scale_kind == WZ_SCALE_F32 || T < 1024) return kPM;
+  const int64_t P = T * d->topk, E = d->n_experts;
+  const int64_t w13_blocks = (P / kPrefillWideRows + std::min(P, E)) * (d->inter / 128);
+  return P >= (d->inter >= 2048 ? 32 : 48) * E && w13_blocks >= 256 ? kPrefillWideRows : kPM;
 }
 
 // A dense MXFP4 linear in tiles: block b = (M-tile b / nblk, N-block b % nblk).
