@@ -124,11 +124,12 @@ def test_running_max_moves(gpu, h, d, s):
 
 
 @pytest.mark.parametrize("h", [16, 32, 48, 64, 80])
-@pytest.mark.parametrize("s", [1, 260])
+@pytest.mark.parametrize("s", [1, 260, 513])
 def test_head_groups_and_empty_blocks(gpu, h, s):
     """Each number of head tiles a workgroup can hold (one, two, four with the last one
-    missing, a second group of one), split over workgroups and not, with blocks that have no
-    valid index first-but-one, in the middle and last: they are skipped and add nothing."""
+    missing, a second group of one), split over workgroups and not (from 512 head groups on),
+    with blocks that have no valid index first-but-one, in the middle and last: they are
+    skipped and add nothing."""
     d, topk = 512, 64 * 6 + 5
     q, kv, sink, idx = _inputs(31 + h + s, 1, s, h, d, 300, topk, invalid=0.3)
     idx[..., 0] = np.maximum(idx[..., 0], 0)
@@ -137,3 +138,27 @@ def test_head_groups_and_empty_blocks(gpu, h, s):
     idx[:, ::4, 384:] = -1
     scale = d ** -0.5
     _check(_run(gpu, q, kv, sink, idx, scale), om.sparse_attn(q, kv, sink, idx, scale))
+
+
+@pytest.mark.parametrize("d", [128, 256])
+@pytest.mark.parametrize("h", [32, 48, 80, 96, 144])
+@pytest.mark.parametrize("s", [1, 257])
+def test_head_groups_of_narrow_heads(gpu, d, h, s):
+    """The same with heads of 128 (a wave per 16 heads past 32) and 256: last groups of one, two
+    and three tiles, the running maximum moving by more than 8, and a NaN query head, whose
+    products and rescales must not reach its neighbours."""
+    topk = 64 * 4 + 5
+    q, kv, sink, idx = _inputs(57 + h + s + d, 1, s, h, d, 300, topk, invalid=0.2)
+    kv = om.bf16_round((kv * (1.0 + 5.0 * (np.arange(300) // 60))[None, :, None]).astype(np.float32))
+    idx.sort(axis=-1)
+    idx[..., 0] = np.maximum(idx[..., 0], 0)
+    idx[:, ::2, 64:128] = -1
+    idx[:, 1::3, 128:] = -1
+    scale = d ** -0.5
+    ref = om.sparse_attn(q, kv, sink, idx, scale)
+    _check(_run(gpu, q, kv, sink, idx, scale), ref)
+    q[:, :, 5] = np.nan
+    got = _run(gpu, q, kv, sink, idx, scale)
+    assert np.isnan(got[:, :, 5]).all()
+    keep = np.arange(h) != 5
+    _check(got[:, :, keep], ref[:, :, keep])

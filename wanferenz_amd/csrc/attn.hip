@@ -98,9 +98,22 @@ __device__ __forceinline__ uint32_t cvt_bf16x2(float a, float b) {
 // partials and sparse_attn_combine_kernel merges them.
 constexpr int kAttnWaves = 8;
 
-template <int D, int HT, bool SPLIT>
-__global__ __launch_bounds__(64 * kAttnWaves, 2) void sparse_attn_kernel(
-    const uint16_t* __restrict__ q, const uint16_t* __restrict__ kv, const float* __restrict__ sink,
+// Row index that an unused entry of a block gets: its byte offset lies past any cache.
+template <int D>
+constexpr int kNoRow = int(0x80000000u / KsLayout<D>::RB);
+
+template <int D, int HT>
+struct AttnLds {
+  alignas(16) uint8_t p[2][16 * HT][64];  // [kc][head]: group g's 8 k slots at 16 g
+  float max[4][64], l[4][64];             // [row tile][head]
+  int bump[kAttnIdxCap / kAttnBlock], used[kAttnIdxCap / kAttnBlock];
+  int idx[kAttnIdxCap];
+  alignas(256) uint8_t ksb[2][KsLayout<D>::BYTES];
+};
+
+template <int D, int HT, bool SPLIT, class Lds>
+__device__ __forceinline__ void sparse_attn_body(
+    Lds& lds, const uint16_t* __restrict__ q, const uint16_t* __restrict__ kv, const float* __restrict__ sink,
     const int32_t* __restrict__ idx, uint16_t* __restrict__ o, float* __restrict__ part, int S, int H, int N, int topk,
     int bps, int nsplit, float scale) {
   using L = KsLayout<D>;
@@ -108,14 +121,15 @@ __global__ __launch_bounds__(64 * kAttnWaves, 2) void sparse_attn_kernel(
   constexpr int NT = D / 16 / kAttnWaves;     // 16-column tiles of O per wave
   constexpr int SHT = HT == 4 ? 2 : 1;        // head tiles of S per wave
   constexpr int NL = L::NG / kAttnWaves;      // loads of a block per wave
-  constexpr int kNoRow = int(0x80000000u / L::RB);  // an unused index: its byte offset lies past any cache
   static_assert(L::NG % kAttnWaves == 0, "a block's loads must split evenly over the waves");
   static_assert(L::RB / 16 >= 16, "the swizzle permutes 16 chunks of a row");
-  __shared__ __align__(1024) uint8_t ksb[2][L::BYTES];
-  __shared__ __align__(16) uint8_t s_p[2][16 * HT][64];  // [kc][head]: group g's 8 k slots at 16 g
-  __shared__ int s_idx[kAttnIdxCap];
-  __shared__ float s_max[4][64], s_l[4][64];  // [row tile][head]
-  __shared__ int s_bump[kAttnIdxCap / kAttnBlock], s_used[kAttnIdxCap / kAttnBlock];
+  auto& ksb = lds.ksb;
+  auto& s_p = lds.p;
+  auto& s_idx = lds.idx;
+  auto& s_max = lds.max;
+  auto& s_l = lds.l;
+  auto& s_bump = lds.bump;
+  auto& s_used = lds.used;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nl = lane & 15, g = lane >> 4;
@@ -144,7 +158,7 @@ __global__ __launch_bounds__(64 * kAttnWaves, 2) void sparse_attn_kernel(
   for (int j = tid; j < nb * kAttnBlock; j += 64 * kAttnWaves) {
     const int v = blk0 * kAttnBlock + j < topk ? ib[j] : -1;
     const bool ok = v >= 0 && v < N;
-    s_idx[j] = ok ? v : kNoRow;
+    s_idx[j] = ok ? v : kNoRow<D>;
     const uint64_t m = __ballot(ok);  // a wave covers one whole block
     if (lane == 0) {
       s_used[j >> 6] = m != 0;
@@ -226,7 +240,7 @@ __global__ __launch_bounds__(64 * kAttnWaves, 2) void sparse_attn_kernel(
       }
     };
     if (has_s) {
-      const uint64_t vmask = __ballot(s_idx[t * kAttnBlock + lane] != kNoRow);
+      const uint64_t vmask = __ballot(s_idx[t * kAttnBlock + lane] != kNoRow<D>);
 #pragma unroll
       for (int h = 0; h < SHT; ++h) sacc[h] = v4f{0.f, 0.f, 0.f, 0.f};
       // K fragments are read kAhead d chunks ahead of their MFMAs
@@ -378,10 +392,233 @@ __global__ __launch_bounds__(64 * kAttnWaves, 2) void sparse_attn_kernel(
       pp[64 + lane] = poisoned ? __builtin_nanf("") : l_run;
     }
 #pragma unroll
-    for (int ht = 0; ht < HT; ++ht)
+    for (int ht = 0; ht < HT; ++ht) {
+      if (HT == 4 && ht == 3 && h0 + 48 >= H) break;  // the fourth tile of three
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt)
         *reinterpret_cast<v4f*>(pp + 128 + int64_t(16 * ht + nl) * D + (wave * NT + nt) * 16 + 4 * g) = acc[ht][nt];
+    }
+  }
+}
+
+// HT: tiles of the largest head group.  A group of fewer (the last one of H = 80 or 96) runs the
+// body of as many, at their Q, products and partials.
+template <int D, int HT, bool SPLIT>
+__global__ __launch_bounds__(64 * kAttnWaves, 2) void sparse_attn_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ kv, const float* __restrict__ sink,
+    const int32_t* __restrict__ idx, uint16_t* __restrict__ o, float* __restrict__ part, int S, int H, int N, int topk,
+    int bps, int nsplit, float scale) {
+  __shared__ AttnLds<D, HT> lds;
+  if constexpr (HT == 4) {
+    const int h0 = int(blockIdx.x / nsplit) % ((H + 63) / 64) * 64;
+    if (H - h0 <= 16)
+      return sparse_attn_body<D, 1, SPLIT>(lds, q, kv, sink, idx, o, part, S, H, N, topk, bps, nsplit, scale);
+    if (H - h0 <= 32)
+      return sparse_attn_body<D, 2, SPLIT>(lds, q, kv, sink, idx, o, part, S, H, N, topk, bps, nsplit, scale);
+  }
+  sparse_attn_body<D, HT, SPLIT>(lds, q, kv, sink, idx, o, part, S, H, N, topk, bps, nsplit, scale);
+}
+
+// The same products with a wave per 16 heads: 4 waves, wave w has heads 64 hq + 16w .. +16 (a wave
+// past H only helps load).  S^T = K Q^T leaves lane (head n, group g) holding rows 16rt + 4g + i,
+// the A operand of O = P V once two row tiles are paired (k slots 0-3: rows 32kc + 4g + i, slots
+// 4-7: rows 32kc + 16 + 4g + i), so P stays in registers and a block costs one barrier instead of
+// two.  Every wave reads all of K and V from LDS for it, which bounds wider heads (D = 512: 512 KB
+// a block, 346 us where the eight waves above take 174), but at D = 128 the eight waves have 16
+// MFMAs each between their barriers.  64 heads of 128, us here / there: 2 x 1024 queries of 300
+// indices 55.6 / 61, 700 of 640 indices 39.8 / 43, decode of one sequence 9.4 / 10.5; 48 heads
+// 52 / 60, 37.8 / 42.6, 9.2 / 9.4.  Up to 32 heads the eight waves win (32: 50 / 38, 37 / 27).
+template <int D, bool SPLIT>
+__global__ __launch_bounds__(256, 1) void sparse_attn_wave_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ kv, const float* __restrict__ sink,
+    const int32_t* __restrict__ idx, uint16_t* __restrict__ o, float* __restrict__ part, int S, int H, int N, int topk,
+    int bps, int nsplit, float scale) {
+  using L = KsLayout<D>;
+  constexpr int KC = D / 32;     // 32-wide d chunks of S
+  constexpr int NT = D / 16;     // 16-column tiles of O
+  constexpr int NL = L::NG / 4;  // loads of a block per wave
+  static_assert(L::NG % 4 == 0, "a block's loads must split evenly over the 4 waves");
+  static_assert(L::RB / 16 >= 16, "the swizzle permutes 16 chunks of a row");
+  __shared__ __align__(1024) uint8_t ksb[2][L::BYTES];
+  __shared__ int s_idx[kAttnIdxCap];
+  __shared__ int s_used[kAttnIdxCap / kAttnBlock];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nl = lane & 15, g = lane >> 4;
+  const int HQ = (H + 63) / 64;
+  const int c = blockIdx.x % nsplit, qh = blockIdx.x / nsplit;
+  const int hq = qh % HQ, bs = qh / HQ, b = bs / S;
+  const int nblk = (topk + kAttnBlock - 1) / kAttnBlock;
+  const int blk0 = c * bps, blk1 = min(blk0 + bps, nblk);
+  const int nb = blk1 - blk0;  // >= 1: the host never launches an empty split
+  const int hg0 = hq * 64 + 16 * wave;
+  const bool active = hg0 < H;  // H % 16 == 0: the whole head group exists
+
+  // Q fragments (B operand of S^T): lane (head nl, group g) holds d 32cc + 8g .. +8
+  v8s_t qb[KC];
+  const uint16_t* const qrow = q + (int64_t(bs) * H + (active ? hg0 : 0) + nl) * D;
+#pragma unroll
+  for (int cc = 0; cc < KC; ++cc) qb[cc] = *reinterpret_cast<const v8s_t*>(qrow + 32 * cc + 8 * g);
+
+  const int32_t* const ib = idx + int64_t(bs) * topk + int64_t(blk0) * kAttnBlock;
+  for (int j = tid; j < nb * kAttnBlock; j += 256) {
+    const int v = blk0 * kAttnBlock + j < topk ? ib[j] : -1;
+    const bool ok = v >= 0 && v < N;
+    s_idx[j] = ok ? v : kNoRow<D>;
+    const uint64_t m = __ballot(ok);  // a wave covers one whole block
+    if (lane == 0) s_used[j >> 6] = m != 0;
+  }
+  __syncthreads();
+  uint32_t todo = uint32_t(__ballot(lane < nb && s_used[min(lane, nb - 1)] != 0));  // nb <= 32
+  const bool poisoned = blk0 == 0 && !(todo & 1u);
+
+  // rows of block t -> ksb[buf], as in sparse_attn_body
+  const __amdgpu_buffer_rsrc_t kv_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(kv + int64_t(b) * N * D), short(0), int(int64_t(N) * L::RB), 0x00020000);
+  const uint32_t ks_lds = lds_addr(&ksb[0][0]);
+  auto issue = [&](int t, int buf) {
+    const int rin = lane / (L::RB / 16), slot = lane % (L::RB / 16);
+    int ri[NL];  // every row index first: the asm loads below order memory accesses
+#pragma unroll
+    for (int j = 0; j < NL; ++j) ri[j] = s_idx[t * kAttnBlock + (j * 4 + wave) * L::RPI + rin];
+#pragma unroll
+    for (int j = 0; j < NL; ++j) {
+      const int gi = j * 4 + wave, row = gi * L::RPI + rin;
+      const uint32_t vo = uint32_t(ri[j]) * L::RB + ((slot ^ L::swz(row)) << 4);
+      load_lds_16(kv_rsrc, __builtin_amdgcn_readfirstlane(ks_lds + buf * L::BYTES + gi * 1024), vo);
+    }
+  };
+  if (todo) issue(__builtin_ctz(todo), 0);
+
+  v4f acc[NT];  // acc[nt][i] = O[head 4g + i][16nt + nl]
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) acc[nt] = v4f{0.f, 0.f, 0.f, 0.f};
+  float m_use = -INFINITY, l_run = 0.0f;  // head nl: running max, this lane's share of the sum
+
+  for (int buf = 0; todo; buf ^= 1) {
+    const int t = __builtin_ctz(todo);
+    todo &= todo - 1;
+    __builtin_amdgcn_s_waitcnt(0);  // this wave's loads of block t have landed
+    __syncthreads();                // ... and every wave's; the other buffer is free
+    if (todo) issue(__builtin_ctz(todo), buf ^ 1);
+    const uint8_t* const ks = ksb[buf];
+    const uint64_t vmask = __ballot(s_idx[t * kAttnBlock + lane] != kNoRow<D>);
+    if (!active) continue;
+
+    // ---- S^T[rows, 16 heads]: sacc[rt][i] = S[row 16rt + 4g + i][head nl] ----
+    // K fragments are read two d chunks ahead of their MFMAs (three buffers)
+    v4f sacc[4];
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt) sacc[rt] = v4f{0.f, 0.f, 0.f, 0.f};
+    v8s_t kf[3][4];
+    auto kload = [&](int cc) {
+#pragma unroll
+      for (int rt = 0; rt < 4; ++rt)
+        kf[cc % 3][rt] = *reinterpret_cast<const v8s_t*>(ks + L::at(16 * rt + nl, 32 * cc + 8 * g));
+    };
+    kload(0);
+    kload(1);
+#pragma unroll
+    for (int cc = 0; cc < KC; ++cc) {
+      if (cc + 2 < KC) kload(cc + 2);
+      __builtin_amdgcn_sched_barrier(0);  // keep the reads two chunks ahead of their use
+#pragma unroll
+      for (int rt = 0; rt < 4; ++rt) sacc[rt] = mfma_bf16_32(kf[cc % 3][rt], qb[cc], sacc[rt]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    float bmax = -INFINITY;
+#pragma unroll
+    for (int rt = 0; rt < 4; ++rt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        sacc[rt][i] = (vmask >> (16 * rt + 4 * g + i)) & 1 ? sacc[rt][i] * scale : -INFINITY;
+        bmax = fmaxf(bmax, sacc[rt][i]);
+      }
+    bmax = fmaxf(bmax, __shfl_xor(bmax, 16, kWave));
+    bmax = fmaxf(bmax, __shfl_xor(bmax, 32, kWave));
+    const bool bump = bmax > m_use + kLazyMax;
+    if (__ballot(bump)) {
+      // nothing accumulated yet for a head without a maximum
+      const float resc = !bump ? 1.0f : (m_use == -INFINITY ? 0.0f : __expf(m_use - bmax));
+      m_use = bump ? bmax : m_use;
+      l_run *= resc;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float r = __shfl(resc, 4 * g + i, kWave);
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) acc[nt][i] *= r;
+      }
+    }
+    v8s_t pa[2];
+#pragma unroll
+    for (int kc = 0; kc < 2; ++kc) {
+      float pv[8];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        pv[i] = sacc[2 * kc][i] == -INFINITY ? 0.0f : __expf(sacc[2 * kc][i] - m_use);
+        pv[4 + i] = sacc[2 * kc + 1][i] == -INFINITY ? 0.0f : __expf(sacc[2 * kc + 1][i] - m_use);
+        l_run += pv[i] + pv[4 + i];
+      }
+      pa[kc] = __builtin_bit_cast(v8s_t, make_uint4(cvt_bf16x2(pv[0], pv[1]), cvt_bf16x2(pv[2], pv[3]),
+                                                    cvt_bf16x2(pv[4], pv[5]), cvt_bf16x2(pv[6], pv[7])));
+    }
+
+    // ---- O[16 heads, D] += P[16 heads, 64 rows] V[64 rows, D] ----
+    // V fragments are read two column tiles ahead of their MFMAs (three buffers)
+    v8s_t vf[3][2];
+    auto vload = [&](int nt) {
+      const int col = 16 * nt + 4 * (nl & 3);
+#pragma unroll
+      for (int kc = 0; kc < 2; ++kc) {
+        const int row = 32 * kc + 4 * g + (nl >> 2);
+        const v4s_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t*)(ks + L::at(row, col)));
+        const v4s_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t*)(ks + L::at(row + 16, col)));
+        vf[nt % 3][kc] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+      }
+    };
+    vload(0);
+    vload(1);
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      if (nt + 2 < NT) vload(nt + 2);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int kc = 0; kc < 2; ++kc) acc[nt] = mfma_bf16_32(pa[kc], vf[nt % 3][kc], acc[nt]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  if (!active) return;
+
+  l_run += __shfl_xor(l_run, 16, kWave);
+  l_run += __shfl_xor(l_run, 32, kWave);
+  if constexpr (!SPLIT) {
+    // normalise by the sum (sink term included): one reciprocal per head, then
+    // products (within 1 fp32 ulp of the quotient, before the bf16 rounding)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int hd = hg0 + 4 * g + i;
+      const float lh = __shfl(l_run, 4 * g + i, kWave), mh = __shfl(m_use, 4 * g + i, kWave);
+      const float inv = poisoned ? __builtin_nanf("") : 1.0f / (lh + __expf(sink[hd] - mh));
+      uint16_t* const orow = o + (int64_t(bs) * H + hd) * D;
+#pragma unroll
+      for (int nt = 0; nt < NT; nt += 2) {
+        const uint32_t pr = cvt_bf16x2(acc[nt][i] * inv, acc[nt + 1][i] * inv);
+        orow[16 * nt + nl] = uint16_t(pr & 0xFFFFu);
+        orow[16 * nt + 16 + nl] = uint16_t(pr >> 16);
+      }
+    }
+  } else {
+    float* const pp = part + int64_t(blockIdx.x) * attn_part_floats(D);
+    if (g == 0) {
+      pp[16 * wave + nl] = m_use;
+      pp[64 + 16 * wave + nl] = poisoned ? __builtin_nanf("") : l_run;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float* const orow = pp + 128 + int64_t(16 * wave + 4 * g + i) * D;
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) orow[16 * nt + nl] = acc[nt][i];
+    }
   }
 }
 
@@ -463,31 +700,38 @@ static inline AttnSplit attn_split(int64_t units, int64_t topk) {
   return {nsplit, bps};
 }
 
-template <int D, int HT>
+// The kernel for H heads: the head tiles of the largest group decide (a group is 64 heads), and
+// heads of 128 in groups of more than two tiles go to a wave per 16 heads.
+template <int D>
 static int launch_attn(const uint16_t* q, const uint16_t* kv, const float* sink, const int32_t* idx, uint16_t* o,
                        float* part, int64_t units, int S, int H, int N, int topk, AttnSplit sp, float scale,
                        hipStream_t stream) {
+  const dim3 grid{unsigned(units * sp.nsplit)};
+#define WZ_ATTN(KERNEL, THREADS)                                                                                   \
+  WZ_LAUNCH("sparse_attn", stream, (KERNEL), grid, dim3(THREADS), 0, q, kv, sink, idx, o, part, S, H, N, topk,     \
+            sp.bps, sp.nsplit, scale)
+#define WZ_ATTN_HEADS(SPLIT)                                                  \
+  do {                                                                        \
+    if (H <= 16)                                                              \
+      WZ_ATTN((sparse_attn_kernel<D, 1, SPLIT>), 64 * kAttnWaves);            \
+    else if (H <= 32)                                                         \
+      WZ_ATTN((sparse_attn_kernel<D, 2, SPLIT>), 64 * kAttnWaves);            \
+    else if constexpr (D == 128)                                              \
+      WZ_ATTN((sparse_attn_wave_kernel<D, SPLIT>), 256);                      \
+    else                                                                      \
+      WZ_ATTN((sparse_attn_kernel<D, 4, SPLIT>), 64 * kAttnWaves);            \
+  } while (0)
   if (sp.nsplit == 1) {
-    WZ_LAUNCH("sparse_attn", stream, (sparse_attn_kernel<D, HT, false>), dim3{unsigned(units)}, dim3(64 * kAttnWaves), 0, q, kv,
-              sink, idx, o, part, S, H, N, topk, sp.bps, 1, scale);
+    WZ_ATTN_HEADS(false);
     return check_launch("sparse_attn");
   }
-  WZ_LAUNCH("sparse_attn", stream, (sparse_attn_kernel<D, HT, true>), dim3{unsigned(units * sp.nsplit)}, dim3(64 * kAttnWaves), 0, q,
-            kv, sink, idx, o, part, S, H, N, topk, sp.bps, sp.nsplit, scale);
+  WZ_ATTN_HEADS(true);
+#undef WZ_ATTN_HEADS
+#undef WZ_ATTN
   if (int rc = check_launch("sparse_attn")) return rc;
   WZ_LAUNCH("sparse_attn_combine", stream, sparse_attn_combine_kernel<D>, dim3{unsigned(units * 16)}, dim3(256), 0,
             part, sink, o, H, sp.nsplit);
   return check_launch("sparse_attn_combine");
-}
-
-// Head tiles of a workgroup: the heads of a group of 64 that exist.
-template <int D>
-static int launch_attn_heads(const uint16_t* q, const uint16_t* kv, const float* sink, const int32_t* idx, uint16_t* o,
-                             float* part, int64_t units, int S, int H, int N, int topk, AttnSplit sp, float scale,
-                             hipStream_t stream) {
-  if (H <= 16) return launch_attn<D, 1>(q, kv, sink, idx, o, part, units, S, H, N, topk, sp, scale, stream);
-  if (H <= 32) return launch_attn<D, 2>(q, kv, sink, idx, o, part, units, S, H, N, topk, sp, scale, stream);
-  return launch_attn<D, 4>(q, kv, sink, idx, o, part, units, S, H, N, topk, sp, scale, stream);
 }
 
 }  // namespace wz
@@ -541,11 +785,11 @@ extern "C" int wz_sparse_attn(const void* q_bf16, const void* kv_bf16, const flo
   uint16_t* o = static_cast<uint16_t*>(o_bf16);
   float* part = static_cast<float*>(workspace);
   if (D == 512)
-    return launch_attn_heads<512>(q, kv, attn_sink, topk_idxs, o, part, units, int(S), int(H), int(N), int(topk), sp,
-                                  softmax_scale, stream);
+    return launch_attn<512>(q, kv, attn_sink, topk_idxs, o, part, units, int(S), int(H), int(N), int(topk), sp,
+                            softmax_scale, stream);
   if (D == 256)
-    return launch_attn_heads<256>(q, kv, attn_sink, topk_idxs, o, part, units, int(S), int(H), int(N), int(topk), sp,
-                                  softmax_scale, stream);
-  return launch_attn_heads<128>(q, kv, attn_sink, topk_idxs, o, part, units, int(S), int(H), int(N), int(topk), sp,
-                                softmax_scale, stream);
+    return launch_attn<256>(q, kv, attn_sink, topk_idxs, o, part, units, int(S), int(H), int(N), int(topk), sp,
+                            softmax_scale, stream);
+  return launch_attn<128>(q, kv, attn_sink, topk_idxs, o, part, units, int(S), int(H), int(N), int(topk), sp,
+                          softmax_scale, stream);
 }
