@@ -1,5 +1,6 @@
 """The tile GEMM (linear_gemm.hip) at its edges: remainders of every tile shape in M and N,
-the shortest and odd K, each scale kind, unaligned and split outputs.
+the shortest and odd K, each scale kind, unaligned and split outputs.  The cases reach every
+compiled tile kernel, which test_tile_shapes.py checks without a GPU.
 
 Every path of a weight form sums in one order, so a row of a wide call must have the bits of
 the same row in a call of up to 16 rows, which the GEMV and skinny kernels serve (those are
@@ -34,9 +35,18 @@ def _weight8(n, k, w_fp32, dev):
 
 
 # (M, N, K): one row past a tile of each height; N of one and of nine 16-column tiles; a single
-# K-block, K-block counts no stage divides, and grids that reach each larger tile shape
+# K-block, K-block counts no stage divides, and grids that reach each larger tile shape.  Narrow
+# calls with power-of-two scales stay on the skinny kernel (17 x 16 x 128)
 ROW_SHAPES = [(17, 16, 128), (33, 144, 384), (65, 272, 640), (100, 4096, 512), (129, 8192, 1024),
-              (257, 16400, 256), (700, 4096, 1152)]
+              (257, 16400, 256), (700, 4096, 1152), (200, 4080, 8064)]
+# MXFP4 rows are staged two K-blocks at a time: K of whole pairs, stages that end half full (an
+# odd number of pairs: 256, 768, 1280) and, with K = 384, what the tile GEMM does not serve
+FP4_SHAPES = [(33, 16, 256), (33, 144, 768), (65, 272, 1280), (31, 20496, 768), (100, 4096, 512),
+              (333, 2048, 4096), (257, 8208, 256), (300, 5136, 768), (700, 4112, 1280), (1030, 8192, 768),
+              (40, 144, 384)]
+# packed weights: K = 1024 is one K-block a slice of the sum, 2048 and 4096 two, 8192 four, others all
+PACKED_SHAPES = [(33, 144, 1024), (100, 4112, 1024), (300, 5136, 1024), (257, 16400, 1024), (520, 32784, 1024),
+                 (300, 32656, 1024), (300, 2064, 4096), (300, 5136, 2048), (1030, 4112, 2048), (200, 272, 640), (200, 4080, 8192)]
 
 
 @pytest.mark.parametrize("act", ["ue8m0", None])
@@ -49,7 +59,7 @@ def test_fp8_rows_have_the_narrow_bits(gpu, M, Nn, K, w_fp32, act):
 
 
 @pytest.mark.parametrize("act", ["ue8m0", None])
-@pytest.mark.parametrize("M,Nn,K", ROW_SHAPES)
+@pytest.mark.parametrize("M,Nn,K", FP4_SHAPES)
 def test_fp4_rows_have_the_narrow_bits(gpu, M, Nn, K, act):
     g = torch.Generator(device="cuda").manual_seed(M)
     w = torch.randint(0, 256, (Nn, K // 2), device=gpu, generator=g, dtype=torch.uint8).view(torch.float4_e2m1fn_x2)
@@ -58,20 +68,23 @@ def test_fp4_rows_have_the_narrow_bits(gpu, M, Nn, K, act):
     assert torch.equal(kernels.fp4_gemm(q, qs, w, ws), _narrow(lambda a, s: kernels.fp4_gemm(a, s, w, ws), q, qs))
 
 
+@pytest.mark.parametrize("act", ["ue8m0", None])
 @pytest.mark.parametrize("w_fp32", [False, True])
-@pytest.mark.parametrize("M,Nn,K", [(33, 144, 1024), (257, 16400, 1024), (520, 32784, 1024), (300, 2064, 4096),
-                                    (1030, 4112, 2048), (200, 272, 640)])
-def test_packed_rows_have_the_narrow_bits(gpu, M, Nn, K, w_fp32):
+@pytest.mark.parametrize("M,Nn,K", PACKED_SHAPES)
+def test_packed_rows_have_the_narrow_bits(gpu, M, Nn, K, w_fp32, act):
     w, ws = _weight8(Nn, K, w_fp32, gpu)
-    lin = kernels.PackedFp8Linear(w, ws)
-    q, qs = _quant(_rows(M, K, gpu), "ue8m0")
+    lin = kernels.PackedFp8Linear(w, ws, act)
+    q, qs = _quant(_rows(M, K, gpu), act)
     y = lin.gemm(q, qs)
     # K outside the GEMV's set sums in one slice on every path: compared over the rows of one M-tile
     ref = _narrow(lin.gemm, q, qs)
     assert torch.equal(y, ref)
 
 
-@pytest.mark.parametrize("M,N0,N1", [(37, 128, 80), (300, 4096, 2064)])
+SPLITS = [(37, 128, 80), (300, 4096, 2064), (300, 32512, 144)]
+
+
+@pytest.mark.parametrize("M,N0,N1", SPLITS)
 def test_unaligned_and_split_outputs(gpu, M, N0, N1):
     """Outputs two bytes past a 16-byte boundary take the scalar stores; the split at N0 and
     the residual add give the unsplit, aligned bits."""

@@ -73,7 +73,8 @@ def test_choice_counts_resident_workgroups(tmp_path, call, tile):
 # K, where both scales are powers of two and N / 16 workgroups fit the 256 CUs; 16 rows otherwise
 @pytest.mark.parametrize("call,skinny", [
     (fp4_rows(16, 32768, 1024, F32), True), (fp4_rows(17, 2048, 4096, E8), True), (fp4_rows(28, 4096, 4096, E8), True),
-    (fp4_rows(29, 4096, 4096, E8), False), (fp4_rows(17, 4112, 4096, E8), False), (fp4_rows(17, 2048, 4096, F32), False),
+    (fp4_rows(29, 4096, 4096, E8), False), (fp4_rows(17, 4112, 4096, E8), False),
+    (fp4_rows(17, 2048, 4096, F32), False),
     (fp4_rows(28, 16, 12288, N.WZ_SCALE_UE8M0_F32), True), (fp4_rows(32, 4096, 2048, E8), True),
     (fp8_rows(16, 32768, 1024, True, F32), True), (fp8_rows(32, 4096, 2048, False, E8), True),
     (fp8_rows(33, 4096, 2048, False, E8), False), (fp8_rows(17, 4096, 2176, False, E8), False),
@@ -84,3 +85,17 @@ def test_rows_of_the_skinny_kernel(tmp_path, call, skinny):
     _, events = record(tmp_path, [call])
     (name,) = [e["name"] for e in events if e["kind"] == "launch"]
     assert ("skinny_gemm_kernel" in name) == skinny, name
+
+
+def test_bit_tests_reach_every_tile_kernel(tmp_path):
+    """The cases that hold the tile GEMM to the narrow kernels' bits (test_gpu_tile_gemm.py)."""
+    from tests.test_gpu_tile_gemm import FP4_SHAPES, PACKED_SHAPES, ROW_SHAPES, SPLITS
+
+    calls = [fp4_rows(*s, a) for s in FP4_SHAPES for a in (E8, F32)]
+    calls += [fp8_rows(*s, w, a) for s in ROW_SHAPES for a in (E8, F32) for w in (False, True)]
+    calls += [packed(*s, w, a) for s in PACKED_SHAPES for a in (E8, F32) for w in (False, True)]
+    compiled, got = selected(tmp_path, calls)
+    assert got == compiled, sorted(compiled - got)
+    # the one tile with two blocks of weight scales along N, with a split output as well
+    (wide,) = [k for k in compiled if k.startswith("wz::TileCfg<8,")]
+    assert wide in selected(tmp_path, [packed(M, a + b, 1024, False) for M, a, b in SPLITS])[1]
