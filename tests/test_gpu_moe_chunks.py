@@ -1,6 +1,7 @@
 """wz_moe_forward's chunks of a long prompt: a layer of many experts takes up to 65536 routed
 pairs at once, a caller whose workspace holds 16384 pairs gets chunks of those.  The layer is
-token-local and every chunk here runs the prefill kernels, so outputs and routing are equal."""
+token-local, so the outputs and routing of chunks that run the prefill kernels are equal; a rest of
+up to 16 tokens runs the decode kernels and is left out of that comparison."""
 
 import ctypes
 import dataclasses
@@ -27,7 +28,7 @@ def _run(moe, x, ws):
 
 
 # 65536 / 6 = 10922 tokens a chunk at 256 experts (64 count workgroups in the permutation), 5461 at
-# 128; one token more than one full chunk would run the decode kernels, so the rest is >= 17
+# 128; the small chunks of 2730 leave 2, 22, 20 and 17 tokens
 @pytest.mark.parametrize("E,T", [(256, 10922), (256, 10942), (128, 5480), (128, 2731 + 16)])
 def test_large_chunks_equal_small_ones(gpu, E, T):
     from tests.test_gpu_moe import upload_case
@@ -41,8 +42,9 @@ def test_large_chunks_equal_small_ones(gpu, E, T):
     assert need > moe.workspace_bytes(small)
     big = _run(moe, x, torch.empty(need, dtype=torch.uint8, device=gpu))
     few = _run(moe, x, torch.empty(moe.workspace_bytes(small), dtype=torch.uint8, device=gpu))
+    n = T - T % small if T % small <= 16 else T
     for a, b in zip(big, few):
-        assert torch.equal(a, b)
+        assert torch.equal(a[:n], b[:n])
     # sampled rows against calls of their own, 32 tokens each
     for t in (0, small - 16, T - 32):
         assert torch.equal(big[0][t:t + 32], moe.forward(x[t:t + 32].contiguous()))
