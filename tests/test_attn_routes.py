@@ -1,4 +1,4 @@
-"""Which sparse attention kernel a call takes, on a recording HIP runtime."""
+"""Which sparse attention kernels a call takes, on a recording HIP runtime."""
 
 import pytest
 
@@ -8,21 +8,30 @@ P = 1 << 20  # a 16-byte aligned stand-in for every operand: nothing is derefere
 BIG = 1 << 40
 
 
-# tiles of 16 heads in the largest group of 64 decide; heads of 128 in more than two tiles take a wave
-# per tile.  From 512 groups on a query's blocks are not split and nothing is merged
-@pytest.mark.parametrize("split", [True, False])
+def _launches(tmp_path, s, h, d):
+    _, events = record(tmp_path, [("wz_sparse_attn", P, P, P, P, P, 1, s, h, d, 1000, 640, 0.1, P, BIG, None)])
+    return [(e["name"].split("(")[0].split("wz::")[1], e["grid"], e["block"]) for e in events if e["kind"] == "launch"]
+
+
+# ten blocks of 64 indices, one workgroup each: 3 queries are split and merged
 @pytest.mark.parametrize("d", [128, 256, 512])
-@pytest.mark.parametrize("h,tiles", [(16, 1), (32, 2), (48, 4), (64, 4), (80, 4), (192, 4)])
-def test_kernel_of_a_shape(tmp_path, h, tiles, d, split):
-    s = 3 if split else 512
-    call = ("wz_sparse_attn", P, P, P, P, P, 1, s, h, d, 1000, 640, 0.1, P, BIG, None)
-    _, events = record(tmp_path, [call])
-    launches = [e for e in events if e["kind"] == "launch"]
-    name = f"sparse_attn_wave_kernel<{d}, {str(split).lower()}>" if d == 128 and tiles == 4 else \
-        f"sparse_attn_kernel<{d}, {tiles}, {str(split).lower()}>"
-    assert name in launches[0]["name"]
-    assert launches[0]["block"] == (256 if "wave" in name else 512)
-    groups = s * ((h + 63) // 64)
-    assert launches[0]["grid"] == groups * (10 if split else 1)
-    assert [e["name"] for e in launches[1:]] == [e["name"] for e in launches if "combine" in e["name"]]
-    assert len(launches) == (2 if split else 1)
+@pytest.mark.parametrize("h,tiles", [(16, 1), (32, 2), (48, 4), (64, 4), (80, 4), (96, 4), (112, 4), (192, 4)])
+def test_split_queries(tmp_path, h, tiles, d):
+    groups = 3 * ((h + 63) // 64)
+    wave = tiles == 4 and d <= 256
+    main = (f"sparse_attn_wave_kernel<{d}, true>", groups * 10, 256) if wave else \
+        (f"sparse_attn_kernel<{d}, {tiles}, true>", groups * 10, 512)
+    assert _launches(tmp_path, 3, h, d) == [main, (f"sparse_attn_combine_kernel<{d}>", groups * 16, 256)]
+
+
+# from 512 groups on a workgroup takes all of a query's blocks; a last group of one or two tiles
+# has a launch of its own
+@pytest.mark.parametrize("d", [128, 256, 512])
+@pytest.mark.parametrize("h,parts", [(16, [(1, 1)]), (32, [(2, 1)]), (48, [(4, 1)]), (64, [(4, 1)]),
+                                     (80, [(4, 1), (1, 1)]), (96, [(4, 1), (2, 1)]), (112, [(4, 2)]),
+                                     (144, [(4, 2), (1, 1)]), (192, [(4, 3)])])
+def test_unsplit_queries(tmp_path, h, parts, d):
+    want = [(f"sparse_attn_kernel<{d}, {tiles}, false>", 512 * groups, 512) for tiles, groups in parts]
+    if d == 128 and h > 32:
+        want = [(f"sparse_attn_wave_kernel<{d}, false>", 512 * ((h + 63) // 64), 256)]
+    assert _launches(tmp_path, 512, h, d) == want

@@ -29,15 +29,15 @@ __device__ __forceinline__ v4f mfma_bf16_32(v8s_t a, v8s_t b, v4f c) {
 // Floats of one (query, 64 heads, split) partial: m[64], l[64], O[64][D].
 __host__ __device__ constexpr int64_t attn_part_floats(int d) { return 128 + 64 * int64_t(d); }
 
-// LDS image of one block of 64 KV rows, row-major, no padding.  The 16-byte
-// chunks of row r sit XOR-swizzled (chunk c at slot c ^ swz(r)) so that both
-// read patterns spread over the banks.  A 16-byte read of one chunk of
-// 16 rows (the K operand of S^T) is served in passes of 16 lanes that mix rows
-// 0-3 and 12-15 of one lane group with rows 4-11 of the next, whose chunk is
-// the neighbour: the slots of rows 0-3 and 12-15 are closed under ^ 1, so the
-// passes' slots are distinct (conflicts took 44 % of the LDS cycles without
-// that, 30 % with it; P's 8-byte writes and the transpose reads are the rest).  The transpose reads of V take two adjacent chunks of 8
-// consecutive rows, which have distinct slot pairs.
+// LDS image of one block of 64 KV rows, row-major, no padding.  The 16-byte chunks of
+// row r sit XOR-swizzled (chunk c at slot c ^ swz(r)) so that both read patterns spread
+// over the banks.  A 16-byte read of one chunk of 16 rows (the K operand of S^T) is
+// served in passes of 16 lanes that mix rows 0-3 and 12-15 of one lane group with rows
+// 4-11 of the next, whose chunk is the neighbour: the slots of rows 0-3 and 12-15 are
+// closed under ^ 1, so the passes' slots are distinct (conflicts took 44 % of the LDS
+// cycles without that, 30 % with it; P's 8-byte writes and the transpose reads are the
+// rest).  The transpose reads of V take two adjacent chunks of 8 consecutive rows,
+// which have distinct slot pairs.
 template <int D>
 struct KsLayout {
   static constexpr int RB = 2 * D;             // bytes per row
@@ -102,20 +102,12 @@ constexpr int kAttnWaves = 8;
 template <int D>
 constexpr int kNoRow = int(0x80000000u / KsLayout<D>::RB);
 
-template <int D, int HT>
-struct AttnLds {
-  alignas(16) uint8_t p[2][16 * HT][64];  // [kc][head]: group g's 8 k slots at 16 g
-  float max[4][64], l[4][64];             // [row tile][head]
-  int bump[kAttnIdxCap / kAttnBlock], used[kAttnIdxCap / kAttnBlock];
-  int idx[kAttnIdxCap];
-  alignas(256) uint8_t ksb[2][KsLayout<D>::BYTES];
-};
-
-template <int D, int HT, bool SPLIT, class Lds>
-__device__ __forceinline__ void sparse_attn_body(
-    Lds& lds, const uint16_t* __restrict__ q, const uint16_t* __restrict__ kv, const float* __restrict__ sink,
+// The launch's workgroups cover head groups hq0 .. hq0 + nhq of every query.
+template <int D, int HT, bool SPLIT>
+__global__ __launch_bounds__(64 * kAttnWaves, 2) void sparse_attn_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ kv, const float* __restrict__ sink,
     const int32_t* __restrict__ idx, uint16_t* __restrict__ o, float* __restrict__ part, int S, int H, int N, int topk,
-    int bps, int nsplit, float scale) {
+    int bps, int nsplit, int hq0, int nhq, float scale) {
   using L = KsLayout<D>;
   constexpr int KC = D / 32;                  // 32-wide d chunks of S
   constexpr int NT = D / 16 / kAttnWaves;     // 16-column tiles of O per wave
@@ -123,19 +115,16 @@ __device__ __forceinline__ void sparse_attn_body(
   constexpr int NL = L::NG / kAttnWaves;      // loads of a block per wave
   static_assert(L::NG % kAttnWaves == 0, "a block's loads must split evenly over the waves");
   static_assert(L::RB / 16 >= 16, "the swizzle permutes 16 chunks of a row");
-  auto& ksb = lds.ksb;
-  auto& s_p = lds.p;
-  auto& s_idx = lds.idx;
-  auto& s_max = lds.max;
-  auto& s_l = lds.l;
-  auto& s_bump = lds.bump;
-  auto& s_used = lds.used;
+  __shared__ __align__(1024) uint8_t ksb[2][L::BYTES];
+  __shared__ __align__(16) uint8_t s_p[2][16 * HT][64];  // [kc][head]: group g's 8 k slots at 16 g
+  __shared__ int s_idx[kAttnIdxCap];
+  __shared__ float s_max[4][64], s_l[4][64];  // [row tile][head]
+  __shared__ int s_bump[kAttnIdxCap / kAttnBlock], s_used[kAttnIdxCap / kAttnBlock];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nl = lane & 15, g = lane >> 4;
-  const int HQ = (H + 63) / 64;
   const int c = blockIdx.x % nsplit, qh = blockIdx.x / nsplit;
-  const int hq = qh % HQ, bs = qh / HQ, b = bs / S;
+  const int hq = hq0 + qh % nhq, bs = qh / nhq, b = bs / S;
   const int nblk = (topk + kAttnBlock - 1) / kAttnBlock;
   const int blk0 = c * bps, blk1 = min(blk0 + bps, nblk);
   const int nb = blk1 - blk0;  // >= 1: the host never launches an empty split
@@ -392,31 +381,11 @@ __device__ __forceinline__ void sparse_attn_body(
       pp[64 + lane] = poisoned ? __builtin_nanf("") : l_run;
     }
 #pragma unroll
-    for (int ht = 0; ht < HT; ++ht) {
-      if (HT == 4 && ht == 3 && h0 + 48 >= H) break;  // the fourth tile of three
+    for (int ht = 0; ht < HT; ++ht)
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt)
         *reinterpret_cast<v4f*>(pp + 128 + int64_t(16 * ht + nl) * D + (wave * NT + nt) * 16 + 4 * g) = acc[ht][nt];
-    }
   }
-}
-
-// HT: tiles of the largest head group.  A group of fewer (the last one of H = 80 or 96) runs the
-// body of as many, at their Q, products and partials.
-template <int D, int HT, bool SPLIT>
-__global__ __launch_bounds__(64 * kAttnWaves, 2) void sparse_attn_kernel(
-    const uint16_t* __restrict__ q, const uint16_t* __restrict__ kv, const float* __restrict__ sink,
-    const int32_t* __restrict__ idx, uint16_t* __restrict__ o, float* __restrict__ part, int S, int H, int N, int topk,
-    int bps, int nsplit, float scale) {
-  __shared__ AttnLds<D, HT> lds;
-  if constexpr (HT == 4) {
-    const int h0 = int(blockIdx.x / nsplit) % ((H + 63) / 64) * 64;
-    if (H - h0 <= 16)
-      return sparse_attn_body<D, 1, SPLIT>(lds, q, kv, sink, idx, o, part, S, H, N, topk, bps, nsplit, scale);
-    if (H - h0 <= 32)
-      return sparse_attn_body<D, 2, SPLIT>(lds, q, kv, sink, idx, o, part, S, H, N, topk, bps, nsplit, scale);
-  }
-  sparse_attn_body<D, HT, SPLIT>(lds, q, kv, sink, idx, o, part, S, H, N, topk, bps, nsplit, scale);
 }
 
 // The same products with a wave per 16 heads: 4 waves, wave w has heads 64 hq + 16w .. +16 (a wave
@@ -700,35 +669,50 @@ static inline AttnSplit attn_split(int64_t units, int64_t topk) {
   return {nsplit, bps};
 }
 
-// The kernel for H heads: the head tiles of the largest group decide (a group is 64 heads), and
-// heads of 128 in groups of more than two tiles go to a wave per 16 heads.
+// The kernel of a shape.  Head groups hold 64 heads, up to four tiles of 16.
+//  * Groups of more than two tiles of narrow heads take a wave per tile: heads of 128, and of 256
+//    where the blocks are split (there 48 heads of one sequence 9.9 / 11.2 us against the eight
+//    waves, 80 of eight with 2048 indices 21.9 / 23.0, 64 of 33 queries 21.7 / 22.6).
+//  * Elsewhere the eight waves are compiled for one, two and four tiles.  The last group of H =
+//    80, 96 or 144 has one or two, and unsplit queries give it a launch of its own with as many
+//    (2 x 1024 queries of 300 indices, 80 heads of 512: 300 us with four tiles for it, 246 so).
 template <int D>
 static int launch_attn(const uint16_t* q, const uint16_t* kv, const float* sink, const int32_t* idx, uint16_t* o,
                        float* part, int64_t units, int S, int H, int N, int topk, AttnSplit sp, float scale,
                        hipStream_t stream) {
-  const dim3 grid{unsigned(units * sp.nsplit)};
-#define WZ_ATTN(KERNEL, THREADS)                                                                                   \
-  WZ_LAUNCH("sparse_attn", stream, (KERNEL), grid, dim3(THREADS), 0, q, kv, sink, idx, o, part, S, H, N, topk,     \
-            sp.bps, sp.nsplit, scale)
-#define WZ_ATTN_HEADS(SPLIT)                                                  \
-  do {                                                                        \
-    if (H <= 16)                                                              \
-      WZ_ATTN((sparse_attn_kernel<D, 1, SPLIT>), 64 * kAttnWaves);            \
-    else if (H <= 32)                                                         \
-      WZ_ATTN((sparse_attn_kernel<D, 2, SPLIT>), 64 * kAttnWaves);            \
-    else if constexpr (D == 128)                                              \
-      WZ_ATTN((sparse_attn_wave_kernel<D, SPLIT>), 256);                      \
-    else                                                                      \
-      WZ_ATTN((sparse_attn_kernel<D, 4, SPLIT>), 64 * kAttnWaves);            \
-  } while (0)
-  if (sp.nsplit == 1) {
-    WZ_ATTN_HEADS(false);
-    return check_launch("sparse_attn");
+  const int HQ = (H + 63) / 64;
+  const bool split = sp.nsplit > 1;
+  const int64_t queries = units / HQ;
+#define WZ_ATTN_EIGHT(HT, SPLIT, HQ0, NHQ)                                                                           \
+  WZ_LAUNCH("sparse_attn", stream, (sparse_attn_kernel<D, HT, SPLIT>), dim3{unsigned(queries * (NHQ) * sp.nsplit)},  \
+            dim3(64 * kAttnWaves), 0, q, kv, sink, idx, o, part, S, H, N, topk, sp.bps, sp.nsplit, HQ0, NHQ, scale)
+#define WZ_ATTN_WAVE(SPLIT)                                                                                          \
+  WZ_LAUNCH("sparse_attn", stream, (sparse_attn_wave_kernel<D, SPLIT>), dim3{unsigned(units * sp.nsplit)},           \
+            dim3(256), 0, q, kv, sink, idx, o, part, S, H, N, topk, sp.bps, sp.nsplit, scale)
+  if (H <= 16) {
+    if (split) WZ_ATTN_EIGHT(1, true, 0, 1); else WZ_ATTN_EIGHT(1, false, 0, 1);
+  } else if (H <= 32) {
+    if (split) WZ_ATTN_EIGHT(2, true, 0, 1); else WZ_ATTN_EIGHT(2, false, 0, 1);
+  } else if (split) {
+    if constexpr (D <= 256)
+      WZ_ATTN_WAVE(true);
+    else
+      WZ_ATTN_EIGHT(4, true, 0, HQ);
+  } else if constexpr (D == 128) {
+    WZ_ATTN_WAVE(false);
+  } else {
+    const int rest = H & 63;
+    const int full = rest != 0 && rest <= 32 ? HQ - 1 : HQ;
+    WZ_ATTN_EIGHT(4, false, 0, full);
+    if (full < HQ) {
+      if (int rc = check_launch("sparse_attn")) return rc;
+      if (rest <= 16) WZ_ATTN_EIGHT(1, false, full, 1); else WZ_ATTN_EIGHT(2, false, full, 1);
+    }
   }
-  WZ_ATTN_HEADS(true);
-#undef WZ_ATTN_HEADS
-#undef WZ_ATTN
+#undef WZ_ATTN_WAVE
+#undef WZ_ATTN_EIGHT
   if (int rc = check_launch("sparse_attn")) return rc;
+  if (!split) return WZ_OK;
   WZ_LAUNCH("sparse_attn_combine", stream, sparse_attn_combine_kernel<D>, dim3{unsigned(units * 16)}, dim3(256), 0,
             part, sink, o, H, sp.nsplit);
   return check_launch("sparse_attn_combine");
