@@ -759,7 +759,7 @@ def cpu_baseline(layers, cfg, T, dev):
 
 
 def committed_mfma_busy():
-    """MFMA busy (%) of the prefill w1/w3 and w2 launches at T = 2048 from the committed
+    """MFMA busy (%) of the routed w1/w3 and w2 launches at T = 2048 from the committed
     rocprofv3 counter summary: the calibrated Zipf batch, then the hot-expert batch."""
     import re
 

@@ -96,7 +96,8 @@ int wz_fp8_linear_packed(const void* x_bf16, const void* w_packed, const void* w
  * decode retile serves it (_fp8_gemm_fast, fp8_vector.py:289-297): M <= 16 with
  * K in {1024, 2048, 4096, 8192} runs the GEMV, otherwise the dense tile GEMM.  ws must
  * hold wz_fp8_gemm_packed_workspace_bytes(M, K, act_scale_kind) bytes (nonzero
- * only for e8m0 activation scales outside the GEMV). */
+ * only for e8m0 activation scales outside the GEMV; asked for at every N, used
+ * where M x K or N x K is past the tile GEMM's 32-bit range or K past 15872). */
 size_t wz_fp8_gemm_packed_workspace_bytes(int64_t M, int64_t K, int act_scale_kind);
 int wz_fp8_gemm_packed(const void* a_e4m3, const void* a_s, const void* w_packed, const void* w_s,
                        void* c_bf16, int64_t M, int64_t N, int64_t K, int act_scale_kind, int w_scale_kind,

@@ -28,9 +28,8 @@ constexpr int kGemmThreads = 256;
 // win up to 32 rows of a K of up to 2048 (skinny / tile us, e4m3 20 x 4096 x 2048 5.6 / 6.2, 32 x
 // 4096 x 1024 4.1 / 4.6, MXFP4 31 x 4096 x 1024 3.9 / 4.3) and, for MXFP4 weights, up to 28 rows of
 // a longer one (17 x 2048 x 4096 7.4 / 8.8, 28 rows 8.6 / 8.8, 32 rows 9.0 / 8.8; e4m3 at K = 4096
-// 17 rows 8.4 / 8.4).  Wider
-// N and float scales go the other way from 17 rows on (17 x 32768 x 1024 e4m3 14.8 / 9.2, MXFP4
-// 12.1 / 6.0; 17 x 4096 x 4096 with float scales 16.2 / 9.3).
+// 17 rows 8.4 / 8.4).  Wider N and float scales go the other way from 17 rows on (17 x 32768 x 1024
+// e4m3 14.8 / 9.2, MXFP4 12.1 / 6.0; 17 x 4096 x 4096 with float scales 16.2 / 9.3).
 static int64_t skinny_max_rows(bool fp4, bool pow2, int64_t N, int64_t K) {
   if (!pow2 || N / 16 > cu_count()) return 16;
   return K <= 2048 ? 32 : fp4 ? 28 : 16;

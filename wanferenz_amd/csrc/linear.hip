@@ -1218,6 +1218,8 @@ static int gemm_packed(const char* name, const void* a_e4m3, const void* a_s, co
   const bool tile = tile_gemm_fits(M, N, K);
   if (y_hi && !tile) return set_error(WZ_EINVAL, "%s: a split output outside the tile GEMM's range", name);
   const float* xs = static_cast<const float*>(a_s);
+  // asked for whenever the size query, which does not know N, states one; the tile GEMM reads e8m0
+  // scales as they are and writes nothing to it, the dense product beyond its range converts them
   if (act_scale_kind == WZ_SCALE_UE8M0) {
     const size_t need = wz_fp8_gemm_packed_workspace_bytes(M, K, act_scale_kind);
     if (!ws || ws_bytes < need)
@@ -1225,7 +1227,6 @@ static int gemm_packed(const char* name, const void* a_e4m3, const void* a_s, co
                        (long long)M, (long long)K, ws_bytes);
   }
   const uint8_t* xq = static_cast<const uint8_t*>(a_e4m3);
-  // the tile GEMM reads e8m0 scales as they are
   if (tile)
     return launch_tile_gemm(xq, a_s, act_scale_kind, w, w_s, w_scale_kind, res, c, y_hi, n_split, M, N, K, stream);
   if (act_scale_kind == WZ_SCALE_UE8M0) {

@@ -420,7 +420,7 @@ static int launch_best(const char* name, const TileArgs& p, bool b_pow2, hipStre
 // with column-major bf16 stores before it.  Where a grid leaves CUs idle the smaller shapes win
 // although they read each operand more often.  At K = 1024 with power-of-two scales (a slice is
 // one K-block, so no second accumulator) 256 x 256 fits: 1999 x 40960 x 1024 in 140 us
-// (1.19 PFLOP/s) against 163 as 128 x 128; before, 381.
+// against 163 as 128 x 128; in a run of passes 115 us (1.46 PFLOP/s), the four-wave kernel 361.
 // Row-major weights against skinny_gemm_kernel, which re-reads the rows once per 16 columns:
 // fp8 100 x 4096 x 4096 33 -> 11.4 us, fp4 333 x 2048 x 4096 59 -> 12.5 us.
 using Sh32 = TileShape<TileCfg<1, 1, 2, 2, 1, 8, 2>, 1, 105, 105>;

@@ -1037,9 +1037,9 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(2))) 
 // the products of q.  Three K-blocks in flight at one workgroup a CU took 1122 us where this
 // takes 831: more waves hide more than more loads.  What bounds it now: half of the wave
 // cycles wait for loads (the experts' weights come from beyond L2), the matrix cores are busy
-// 40 %.  M-tiles in order, each with all its N-blocks (788 us for w1/w3 against 838 in groups
+// 44 %.  M-tiles in order, each with all its N-blocks (788 us for w1/w3 against 838 in groups
 // of 8 x 8).  6000 tokens over 256 experts, w1/w3 and w2 with the shared expert: 1061 + 574 ->
-// 955 + 451 us, the layer 1840 -> 1553; 2048 tokens with skewed experts 920 -> 863.
+// 955 + 451 us, the layer 1840 -> 1600; 2048 tokens with skewed experts 920 -> 867.
 constexpr int kWideThreads = 512;
 constexpr int kWideStage = kPrefillWideRows * 128 + 16 * 1024;  // rows, then 16 weight tiles
 constexpr int kWideScales = 16 * 256;                           // weight scales of 4 K-blocks
