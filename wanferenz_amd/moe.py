@@ -565,7 +565,8 @@ def prepare(module, mod=None, max_tokens: int = 16) -> int:
     """Pack every MoE layer of ``module`` that the HIP path serves, now (at load,
     before any graph capture), with a workspace for ``max_tokens``: the role of
     the reference's load-time bank layout (serving/partition.py:398-405), so the
-    first captured step allocates nothing.  Returns the number of layers packed."""
+    first captured step of up to CHUNK_PAIRS routed pairs allocates nothing.
+    Returns the number of layers packed."""
     mod = mod or _MOD
     n = 0
     for m in module.modules():
